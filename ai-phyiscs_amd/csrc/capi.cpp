@@ -294,6 +294,12 @@ int chysx_cloth_step(chysx_cloth* sim, float dt, uintptr_t stream) {
         sim->sim.step(dt, stream);
     });
 }
+int chysx_cloth_set_resident_solve(chysx_cloth* sim, int mode) {
+    return guard([&] {
+        need(sim, "simulator");
+        sim->sim.problem().set_resident_solve(mode);
+    });
+}
 int chysx_cloth_set_pin_projection(chysx_cloth* sim, int on) {
     return guard([&] {
         need(sim, "sim");
@@ -533,6 +539,12 @@ int chysx_batch_set_split_advance(chysx_batch* b, int mode) {
     return guard([&] {
         need(b, "batch");
         b->batch.problem().set_split_advance(mode);
+    });
+}
+int chysx_batch_set_resident_solve(chysx_batch* b, int mode) {
+    return guard([&] {
+        need(b, "batch");
+        b->batch.problem().set_resident_solve(mode);
     });
 }
 int chysx_batch_set_pin_projection(chysx_batch* b, int on) {

@@ -27,6 +27,7 @@
 
 #include "cloth_kernels.hpp"
 #include "matrix_access.hpp"
+#include "pcg_device.hpp"
 
 namespace chysx_amd {
 
@@ -34,7 +35,6 @@ namespace {
 
 constexpr float kMinLength = 1.0e-6f;  // spring_constraint.cu:35
 constexpr float kMinNorm = 1.0e-6f;    // triangle_stretch_constraint.cu:39
-constexpr double kGuard = 1.0e-37;     // pcg_solver.cu:421-423,451
 constexpr size_t kAssembleLdsBytes = 64 * 1024;
 
 // Slice owned by this wavefront (>= nslices: nothing to do).
@@ -52,40 +52,6 @@ inline int grid_for(int nslices, int waves) {
     const int nwg = (nslices + waves - 1) / waves;
     return 8 * ((nwg + 7) / 8);
 }
-
-struct F3 {
-    float x, y, z;
-};
-__device__ __forceinline__ F3 f3(float x, float y, float z) { return {x, y, z}; }
-__device__ __forceinline__ F3 operator+(F3 a, F3 b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }
-__device__ __forceinline__ F3 operator-(F3 a, F3 b) { return {a.x - b.x, a.y - b.y, a.z - b.z}; }
-__device__ __forceinline__ F3 operator*(F3 a, float s) { return {a.x * s, a.y * s, a.z * s}; }
-__device__ __forceinline__ float dot(F3 a, F3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
-__device__ __forceinline__ F3 ld3(const float* p, int i) { return {p[3 * i], p[3 * i + 1], p[3 * i + 2]}; }
-__device__ __forceinline__ void st3(float* p, int i, F3 v) {
-    p[3 * i] = v.x;
-    p[3 * i + 1] = v.y;
-    p[3 * i + 2] = v.z;
-}
-
-// Symmetric 3x3 (xx, xy, xz, yy, yz, zz).
-// a + (m0 p.x + m1 p.y + m2 p.z) as one fixed chain of FMAs.  Written out so
-// that every kernel variant (unroll, padding mode, storage) rounds the same
-// way whatever the compiler schedules.
-__device__ __forceinline__ float fma3(float a, float m0, float m1, float m2, F3 p) {
-    return fmaf(m2, p.z, fmaf(m1, p.y, fmaf(m0, p.x, a)));
-}
-__device__ __forceinline__ double fma3d(double a, double m0, double m1, double m2, double x0, double x1, double x2) {
-    return fma(m2, x2, fma(m1, x1, fma(m0, x0, a)));
-}
-// z + beta p_prev, component-wise FMAs
-__device__ __forceinline__ F3 dir3(F3 z, F3 pp, float beta) {
-    return F3{fmaf(pp.x, beta, z.x), fmaf(pp.y, beta, z.y), fmaf(pp.z, beta, z.z)};
-}
-
-struct S6 {
-    float m[6];
-};
 
 // Workgroup of kGroupSlices wavefronts (one 16-slice group): wave sums, then
 // the 16 waves in order; thread j < N writes slot slot[j] of `group`.  Every
@@ -682,12 +648,6 @@ __global__ __launch_bounds__(64 * WAVES) void assemble_kernel(LaunchGeom g, DevM
     mv[5 * 64] = a22 * id;
 }
 
-__device__ __forceinline__ F3 minv_mul(const DevMatrix& A, int s, int lane, F3 r) {
-    const float* mv = A.minv + (size_t)s * 6 * 64 + lane;
-    const float m0 = mv[0], m1 = mv[64], m2 = mv[128], m3 = mv[192], m4 = mv[256], m5 = mv[320];
-    return f3(fma3(0.0f, m0, m1, m2, r), fma3(0.0f, m1, m3, m4, r), fma3(0.0f, m2, m4, m5, r));
-}
-
 constexpr int kReduceThreads = 64 * kGroupSlices;
 
 // Sums slots slot[0..NS) of an instance's group partials (groups g0 ..
@@ -805,74 +765,18 @@ __device__ __forceinline__ double wave_group_sum(const double* __restrict__ p, i
 }
 
 // ---------------------------------------------------------------------------
-// ---------------------------------------------------------------------------
-// True residual of one row: b - A x with FP64 products and sums (x is FP64).
-// Returns it and, unless `report_only`, stores r, z = M^-1 r and p = z.
+// One row of a residual or check pass: the true residual and, unless
+// `report_only`, r, z = M^-1 r and p = z stored.
 // Partials: [0] |r|^2, [1] |b|^2, [2] r . z.
-// Entries per load batch of residual_row: two keeps both the residual kernel
-// and the SpMV kernel (whose check mode runs residual_row) at 64 VGPRs or
-// fewer, 8 waves per SIMD.
-constexpr int kResidualBatch = 2;
-
-// nlow: the slice's nlower (entries at positions >= nlow hold no lower block
-// in any lane, so their mirror index is not read).
 __device__ __forceinline__ void residual_row(const DevMatrix& A, const DevVectors& v, float* __restrict__ pcur,
                                              int row, int nlow, bool report_only, double (&part)[4]) {
-    const int s = row >> 6, lane = row & 63;
-    const double* x = v.x;
-    float dm[9];
-    load_diag(A, s, lane, dm);
-    const double x0 = x[3 * row], x1 = x[3 * row + 1], x2 = x[3 * row + 2];
-    double a0 = fma3d(0.0, dm[0], dm[1], dm[2], x0, x1, x2);
-    double a1 = fma3d(0.0, dm[3], dm[4], dm[5], x0, x1, x2);
-    double a2 = fma3d(0.0, dm[6], dm[7], dm[8], x0, x1, x2);
-    const int sb = A.slice_ptr[s], w = A.slice_ptr[s + 1] - sb;
-    const int* colp = A.col + (size_t)sb * 64 + lane;
-    const int* mirp = A.mir + (size_t)sb * 64 + lane;
-    const float* vp = A.val + (size_t)sb * A.bs * 64 + lane;
-    // Batches of entries in three phases (the column and mirror indices, then
-    // every block and x gather, then the FP64 FMAs in entry order, so the sums
-    // are those of one entry at a time), so a batch costs two memory round
-    // trips instead of three per entry.
-    constexpr int RB = kResidualBatch;
-    for (int k0 = 0; k0 < w; k0 += RB) {
-        int c[RB], mi[RB];
-#pragma unroll
-        for (int u = 0; u < RB; ++u) {
-            c[u] = -1;
-            mi[u] = 0;
-            if (k0 + u < w) {  // wave-uniform
-                c[u] = colp[(k0 + u) * 64];
-                if (A.sym && k0 + u < nlow) mi[u] = mirp[(k0 + u) * 64];  // wave-uniform
-            }
-        }
-        float m[RB][9];
-        double y[RB][3];
-#pragma unroll
-        for (int u = 0; u < RB; ++u) {
-            if (c[u] >= 0) {
-                load_block_at(A, vp + (k0 + u) * A.bs * 64, mi[u], c[u], row, m[u]);
-                y[u][0] = x[3 * c[u]];
-                y[u][1] = x[3 * c[u] + 1];
-                y[u][2] = x[3 * c[u] + 2];
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < RB; ++u) {
-            if (c[u] >= 0) {
-                a0 = fma3d(a0, m[u][0], m[u][1], m[u][2], y[u][0], y[u][1], y[u][2]);
-                a1 = fma3d(a1, m[u][3], m[u][4], m[u][5], y[u][0], y[u][1], y[u][2]);
-                a2 = fma3d(a2, m[u][6], m[u][7], m[u][8], y[u][0], y[u][1], y[u][2]);
-            }
-        }
-    }
-    const F3 bf = ld3(v.rhs, row);
-    const double r0 = double(bf.x) - a0, r1 = double(bf.y) - a1, r2 = double(bf.z) - a2;
-    part[0] = fma3d(0.0, r0, r1, r2, r0, r1, r2);
+    double r[3];
+    const F3 bf = true_residual<false>(A, v, row >> 6, row & 63, nlow, r);
+    part[0] = fma3d(0.0, r[0], r[1], r[2], r[0], r[1], r[2]);
     part[1] = fma3d(0.0, bf.x, bf.y, bf.z, bf.x, bf.y, bf.z);
     if (!report_only) {
-        const F3 rf = f3(float(r0), float(r1), float(r2));
-        const F3 zf = minv_mul(A, s, lane, rf);
+        const F3 rf = f3(float(r[0]), float(r[1]), float(r[2]));
+        const F3 zf = minv_mul(A, row >> 6, row & 63, rf);
         st3(v.r, row, rf);
         st3(v.z, row, zf);
         st3(pcur, row, zf);
@@ -947,84 +851,6 @@ __global__ __launch_bounds__(64 * kGroupSlices) void pcg_start_given_r_kernel(La
 // so this pass computes the true residual instead.  Mode kModeFlush: the
 // owed iterate term is added.
 // ---------------------------------------------------------------------------
-// Entry order of the symmetric pass: 0, w-1, 1, w-2, ...  A row's columns
-// ascend, so step t pairs its t-th lower entry with its t-th upper entry
-// counted from the end.  On a grid, the mirror that step t reads for lower
-// entry t (row i - W, i - W + 1 or i - 1) is the upper entry that its owner
-// row, 16 slices earlier at W = 1024, streams at its own step t: both
-// wavefronts touch the block at the same point of their lives, a fraction of
-// a microsecond apart, while it is still in L2.  (In ascending order the
-// mirror is read first and the owner reads it at the end of its loop, after
-// the XCD has streamed several L2 capacities.)
-__device__ __forceinline__ int sym_order(int k, int w) { return (k & 1) ? w - 1 - (k >> 1) : (k >> 1); }
-
-// ---------------------------------------------------------------------------
-// Advance of an instance's solver state by one SpMV/update pair, given the
-// sums of the partials that pair wrote: r . z and |r|^2 of the update pass
-// (Iter), or the true ones of the check pass (Check); none for a flush.  Scalar logic restates
-// reduce_rho_beta_kernel (pcg_solver.cu:436-454) with its 1e-37 guard, plus
-// the stopping rule: true relative residual sqrt(|b-Ax|^2 / max(|b|^2,1e-30))
-// <= tol (pcg_solver.cu:595-641, 916-923), or exactly max_iter iterations
-// when tol == 0 (pcg_solver.cu:542-592).  Runs in the next SpMV pass (every
-// workgroup, identical inputs and order) or in pcg_advance_kernel.
-// ---------------------------------------------------------------------------
-struct AdvanceSums {
-    double rz;  // r . z
-    double rr;  // |r|^2
-};
-__device__ __forceinline__ void pcg_advance(InstState& S, const InstParams& pr, const AdvanceSums& t) {
-    const double tol2 = pr.tol2;
-    if (S.mode == kModeFlush) {  // x is whole again
-        S.pend = 0;
-        S.alpha_pend = 0.0;
-        S.defer = 1;
-        if (S.flush_to == kModeCheck) {
-            S.mode = kModeCheck;
-        } else {
-            S.mode = kModeIter;
-            S.status = kStopped;
-        }
-    } else if (S.mode == kModeCheck) {
-        const double rr = t.rr;
-        S.rr = rr;
-        S.relres = sqrt(rr / S.bb);
-        if (rr <= tol2 * S.bb) {
-            S.status = kConverged;
-        } else {  // residual replacement: restart the recursion from b - A x
-            S.restarts += 1;
-            S.rho = t.rz;
-            S.beta = 0.0;
-            S.mode = kModeIter;
-            S.defer = 1;
-            if (S.iters >= pr.max_iter) S.status = kStopped;
-        }
-    } else {
-        const double rho = S.rho, rho_new = t.rz;
-        if (S.pend) {  // this update pass added the owed term
-            S.pend = 0;
-        } else if (S.defer) {  // this update pass left x += alpha p to the next
-            S.alpha_pend = S.alpha;  // the alpha that pass used
-            S.pend = 1;
-        }
-        S.defer = S.pend ? 0 : 1;
-        S.beta = (rho > kGuard || rho < -kGuard) ? rho_new / rho : 0.0;
-        S.rho = rho_new;
-        S.rr = t.rr;
-        S.parity ^= 1;
-        S.iters += 1;
-        const bool check = tol2 > 0.0 && t.rr <= tol2 * S.bb;
-        const bool stop = !check && S.iters >= pr.max_iter;
-        if ((check || stop) && S.pend) {  // complete x first
-            S.mode = kModeFlush;
-            S.flush_to = check ? int(kModeCheck) : int(kStopped);
-        } else if (check) {
-            S.mode = kModeCheck;
-        } else if (stop) {
-            S.status = kStopped;
-        }
-    }
-}
-
 // Sums the partials an owed advance needs (by the whole workgroup, in the
 // fixed order of block_sum; every thread gets the totals).
 __device__ __forceinline__ AdvanceSums advance_sums(const double* __restrict__ partials, int ngroups,
@@ -1047,13 +873,6 @@ __device__ __forceinline__ AdvanceSums advance_sums(const double* __restrict__ p
 // compute the same state; the workgroup of the instance's first group writes
 // it to st_out, for the update pass and the next SpMV pass (also when the
 // instance is not running, so both buffers agree once it has stopped).
-__device__ __forceinline__ int uniform_int(int x) { return __builtin_amdgcn_readfirstlane(x); }
-__device__ __forceinline__ double uniform_double(double x) {
-    const unsigned long long b = static_cast<unsigned long long>(__double_as_longlong(x));
-    const unsigned lo = unsigned(__builtin_amdgcn_readfirstlane(int(unsigned(b))));
-    const unsigned hi = unsigned(__builtin_amdgcn_readfirstlane(int(unsigned(b >> 32))));
-    return __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
-}
 __device__ __forceinline__ void advance_in_pass(const LaunchGeom& g, const DevVectors& v, InstState& S,
                                                 const InstParams* __restrict__ params, InstState* __restrict__ st_out,
                                                 int inst, int grp) {
@@ -1174,9 +993,9 @@ __global__ __launch_bounds__(64 * kGroupSlices) __attribute__((amdgpu_num_sgpr(8
             const F3 pk = ld3(parity ? v.p1 : v.p0, row);
             const double ap = S.alpha_pend;
             double* x = v.x + 3 * row;
-            x[0] += ap * double(pk.x);
-            x[1] += ap * double(pk.y);
-            x[2] += ap * double(pk.z);
+            x[0] = fma(ap, double(pk.x), x[0]);
+            x[1] = fma(ap, double(pk.y), x[1]);
+            x[2] = fma(ap, double(pk.z), x[2]);
         }
         return;
     }
@@ -1336,21 +1155,20 @@ __device__ __forceinline__ void update_rows(const LaunchGeom& g, const DevVector
     if (lane < sd.nvalid) {
         if (X == 1) {  // the owed term and this one
             const double ap = S.alpha_pend;
-            n0 = x0 + (ap * double(pp.x) + alpha * double(pi.x));
-            n1 = x1 + (ap * double(pp.y) + alpha * double(pi.y));
-            n2 = x2 + (ap * double(pp.z) + alpha * double(pi.z));
+            n0 = x_two(x0, ap, pp.x, alpha, pi.x);
+            n1 = x_two(x1, ap, pp.y, alpha, pi.y);
+            n2 = x_two(x2, ap, pp.z, alpha, pi.z);
         } else if (X == 2) {
-            n0 = x0 + alpha * double(pi.x);
-            n1 = x1 + alpha * double(pi.y);
-            n2 = x2 + alpha * double(pi.z);
+            n0 = fma(alpha, double(pi.x), x0);
+            n1 = fma(alpha, double(pi.y), x1);
+            n2 = fma(alpha, double(pi.z), x2);
         }
-        const F3 ri = r0 - api * af;
-        const F3 zi = f3(m[0] * ri.x + m[1] * ri.y + m[2] * ri.z, m[1] * ri.x + m[3] * ri.y + m[4] * ri.z,
-                         m[2] * ri.x + m[4] * ri.y + m[5] * ri.z);
+        const F3 ri = r_update(r0, api, af);
+        const F3 zi = z_update(m, ri);
         st3(v.r, row, ri);
         st3(v.z, row, zi);
-        part[0] = double(ri.x) * zi.x + double(ri.y) * zi.y + double(ri.z) * zi.z;
-        part[1] = double(ri.x) * ri.x + double(ri.y) * ri.y + double(ri.z) * ri.z;
+        part[0] = dot3d(ri, zi);
+        part[1] = dot3d(ri, ri);
     }
     if (X != 0) {
         // the rows' x go out through the wave's slab, each store covering 512 contiguous bytes
@@ -1501,21 +1319,8 @@ __global__ __launch_bounds__(64) void pcg_reduce_kernel(InstState* __restrict__ 
         for (int q = int(threadIdx.x); q < ng; q += 64) gactive[g0 + q] = run ? 1 : 0;
     }
     if (threadIdx.x != 0) return;
-    const double tol2 = pr.tol2;
     if (phase == kPhaseStart) {
-        S.bb = fmax(tot[1], 1.0e-30);
-        S.rr = tot[0];
-        S.relres = sqrt(tot[0] / S.bb);
-        S.iters = 0;
-        S.restarts = 0;
-        S.mode = kModeIter;
-        S.beta = 0.0;
-        S.rho = tot[2];
-        S.pend = 0;
-        S.alpha_pend = 0.0;
-        S.defer = 1;
-        S.owed = 0;
-        S.status = (tol2 > 0.0 && tot[0] <= tol2 * S.bb) ? kConverged : (pr.max_iter <= 0 ? kStopped : kRunning);
+        pcg_begin(S, pr, tot[0], tot[1], tot[2]);
     } else {
         S.rr = tot[0];
         S.relres = sqrt(tot[0] / S.bb);
@@ -1537,18 +1342,7 @@ __global__ __launch_bounds__(64 * WAVES) void finalize_kernel(LaunchGeom g, DevV
     if (lane >= sd.nvalid) return;
     const int row = s * 64 + lane, p = sd.part0 + lane;
     const InstParams pr = params[sd.inst];
-    F3 d = f3(float(v.x[3 * row]), float(v.x[3 * row + 1]), float(v.x[3 * row + 2]));
-    const F3 xn = ld3(e.pos, p);
-    F3 xnew = xn + d;
-    if (pr.pin_proj && pin_inc_off[row + 1] > pin_inc_off[row]) {  // a projected pin ends at its target
-        xnew = ld3(pin_tgt, pin_inc[pin_inc_off[row]]);
-        d = xnew - xn;
-    }
-    const float inv_dt = 1.0f / dt;
-    F3 vn = d * inv_dt;
-    if (pr.damping > 0.0f) vn = vn * expf(-pr.damping * dt);
-    st3(e.pos, p, xnew);
-    st3(e.vel, p, vn);
+    finalize_row(e, pr, dt, pin_inc_off, pin_inc, pin_tgt, row, p, v.x[3 * row], v.x[3 * row + 1], v.x[3 * row + 2]);
 }
 
 // Plain y = A x on the ELL layout (spmv_kernel, block_csr.cu:54-83, alpha=1, beta=0).

@@ -60,6 +60,11 @@ template class DeviceArray<SliceDesc>;
 template class DeviceArray<InstState>;
 template class DeviceArray<InstParams>;
 template class DeviceArray<WsInst>;
+template class DeviceArray<ResidentWg>;
+template class DeviceArray<uint16_t>;
+template class DeviceArray<uint8_t>;
+template class DeviceArray<unsigned long long>;
+template class DeviceArray<ResidentSync>;
 
 // ---------------------------------------------------------------------------
 // Rest data
@@ -481,10 +486,81 @@ void Problem::build(const std::vector<const Instance*>& insts) {
     check_hip(hipHostMalloc(reinterpret_cast<void**>(&host_states_), sizeof(InstState) * std::max(ninst_, 1)),
               "hipHostMalloc(states)");
     std::memcpy(host_states_, st.data(), sizeof(InstState) * st.size());
+    make_resident(sell_col);
     check_hip(hipStreamSynchronize(s), "hipStreamSynchronize(build)");
     stats_.assign(size_t(ninst_), SolveStats());
     last_iters_ = 0;
     built_ = true;
+}
+
+void Problem::make_resident(const std::vector<int>& cols) {
+    res_ = ResidentView{};
+    int dev = 0, cus = 0, lds = 0;
+    check_hip(hipGetDevice(&dev), "hipGetDevice");
+    check_hip(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute(CUs)");
+    check_hip(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev),
+              "hipDeviceGetAttribute(LDS)");
+    std::vector<ResidentInstance> insts(static_cast<size_t>(ninst_));
+    for (int k = 0; k < ninst_; ++k) {
+        insts[size_t(k)].slice0 = inst_slice0_[size_t(k)];
+        insts[size_t(k)].nslices = (inst_n_[size_t(k)] + kSlice - 1) / kSlice;
+    }
+    const ResidentPlan P = plan_resident(insts, slice_ptr_h_, cols, block_floats(), std::min(cus, kResidentMaxWgs),
+                                         lds - kResidentStaticLds);
+    if (P.variant == kResidentNone || P.wgs.empty()) return;
+    hipStream_t s = nullptr;
+    res_wgs_.assign(P.wgs.data(), P.wgs.size(), s);
+    res_loc_.assign(P.loc.data(), P.loc.size(), s);
+    res_halo_.assign(P.halo.data(), P.halo.size(), s);
+    res_exported_.assign(P.exported.data(), P.exported.size(), s);
+    res_sync_.resize(size_t(ninst_));
+    res_ticket_.resize(1);
+    res_zx_.resize(P.max_cluster > 1 ? size_t(n_pad_) * 2 : 1);
+    res_slots_.resize(P.max_cluster > 1 ? resident_slot_words(nslices() / kGroupSlices) : 1);
+    res_solo_.resize(P.max_cluster > 1 ? size_t(nslices()) * 3 : 1);
+    res_sync_.zero(s);
+    res_ticket_.zero(s);
+    res_zx_.zero(s);
+    res_slots_.zero(s);
+    check_hip(hipStreamSynchronize(s), "hipStreamSynchronize(resident plan)");
+    res_.waves = P.waves;
+    res_.block_waves = P.max_cluster > 1 ? P.waves : P.max_nslices;
+    res_.nwg = int(P.wgs.size());
+    res_.lds_rows = P.lds_rows;
+    res_.lds_x = resident_lds_x(P.lds_rows, P.max_halo);
+    res_.lds_bytes = resident_lds_bytes(P.lds_rows, P.max_halo, res_.block_waves);
+    res_.max_cluster = P.max_cluster;
+    res_.wgs = res_wgs_.data();
+    res_.loc = res_loc_.data();
+    res_.halo = res_halo_.data();
+    res_.exported = res_exported_.data();
+    res_.zx = res_zx_.data();
+    res_.rows = n_pad_;
+    res_.slots = res_slots_.data();
+    res_.solo = res_solo_.data();
+    res_.sync = res_sync_.data();
+    res_.ticket = res_ticket_.data();
+    res_.meet_polls = kResidentMeetPolls;
+    res_.variant = P.variant;
+}
+
+void Problem::launch_resident(float dt, const DevExt& ext, hipStream_t s) {
+    ResidentView R = res_;
+    if (res_mode_ == 2) R.meet_polls = 0;
+    const int given_r = start_r_ready_ ? 1 : 0;
+    start_r_ready_ = false;
+    with_resident_gate(R.max_cluster, s, [&] {
+        launch_pcg_resident(R, geom(), matrix(), vectors(), ext, mesh(), state_.data(), host_states_, params_.data(),
+                            dt, given_r, s);
+    });
+}
+
+void Problem::check_resident() const {
+    for (int k = 0; k < ninst_; ++k)
+        if (host_states_[k].status != kConverged && host_states_[k].status != kStopped) {
+            res_mode_ = 0;  // the exchange words are in no known state
+            throw std::runtime_error("PCG: a solve lost one of its workgroups");
+        }
 }
 
 void Problem::upload_params(const std::vector<const Instance*>& insts, hipStream_t s) {
@@ -659,6 +735,10 @@ void Problem::set_launch_config(const LaunchConfig& c) {
         val_.zero(nullptr);
         diag_.zero(nullptr);
         check_hip(hipStreamSynchronize(nullptr), "hipStreamSynchronize(storage change)");
+        std::vector<int> cols(col_.size());
+        check_hip(hipMemcpy(cols.data(), col_.data(), sizeof(int) * cols.size(), hipMemcpyDeviceToHost),
+                  "hipMemcpy(columns)");
+        make_resident(cols);
     }
 }
 
@@ -1032,6 +1112,13 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
     proj_ran_ = false;
     start_r_ready_ = false;
     const bool ws_on = ws_mode_ != kWarmPrevious || ws_train_;
+    if (resident()) {
+        // the solve is launched directly, not as a graph, so a capture is refused here
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        check_hip(hipStreamIsCapturing(s, &capturing), "hipStreamIsCapturing");
+        if (capturing != hipStreamCaptureStatusNone)
+            throw std::runtime_error("step: the stream is being captured; a step cannot be part of a graph");
+    }
     // Every instance at a fixed iteration count (tol == 0): the number of
     // rounds is known, so the whole solve is enqueued without a poll.
     bool fixed = !ws_on && !params_h_.empty();
@@ -1047,7 +1134,11 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
         // long fixed solves replay the chunk graphs instead, so a graph never
         // holds more than kStepGraphMaxChunks chunks
         const int chunks = std::max(1, (fixed_iters + 2 + kChunkIters - 1) / kChunkIters);
-        if (chunks <= kStepGraphMaxChunks) {
+        resident_step_ = resident();
+        if (resident_step_) {
+            launch_assemble(dt, ext, s);
+            launch_resident(dt, ext, s);
+        } else if (chunks <= kStepGraphMaxChunks) {
             launch_fixed_step_graph(dt, ext, chunks, s);
         } else {
             launch_assemble(dt, ext, s);
@@ -1069,6 +1160,16 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
     }
     launch_assemble(dt, ext, s);
     if (ws_on && hist_n_ >= 2) warm_start_stage(dt, ext, s);
+    if (resident()) {
+        launch_resident(dt, ext, s);
+        check_hip(hipStreamSynchronize(s), "hipStreamSynchronize(solve)");
+        check_resident();
+        last_iters_ = 0;
+        for (int k = 0; k < ninst_; ++k) last_iters_ = std::max(last_iters_, host_states_[k].iters);
+        train_after_solve(ws_on, s);
+        end_step(s);
+        return;
+    }
     launch_pcg_start(s);
     // Launch as many rounds as the previous step used (its iterations plus a
     // flush and a check round) before the first poll; rounds after
@@ -1093,6 +1194,15 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
         launch_pcg_reduce(state_.data(), params_.data(), partials_.data(), ninst_, geom().ngroups, kPhaseFinal, s);
         read_states(s);
     }
+    train_after_solve(ws_on, s);
+    launch_finalize(dt, ext, s);
+    end_step(s);
+    last_iters_ = max_it;
+}
+
+// What follows the solve of a warm-started step: the training step on the
+// converged iterate, and the history of solutions.
+void Problem::train_after_solve(bool ws_on, hipStream_t s) {
     if (ws_ran_ && ws_train_) {
         WarmStartNet& N = net();
         const WsReduce red = ws_reduce();
@@ -1103,7 +1213,9 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
         N.adam_step(ws_lr_, s);
     }
     if (ws_on) push_history(s);
-    launch_finalize(dt, ext, s);
+}
+
+void Problem::end_step(hipStream_t s) {
     if (ws_ran_ || proj_ran_) {
         check_hip(hipMemcpyAsync(ws_host_.data(), ws_inst_.data(), sizeof(WsInst) * ninst_, hipMemcpyDeviceToHost, s),
                   "hipMemcpyAsync(warm start stats)");
@@ -1115,7 +1227,6 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
         for (int k = 0; k < ninst_; ++k) l += ws_host_[size_t(k)].loss;
         ws_loss_ = l / double(ninst_);
     }
-    last_iters_ = max_it;
 }
 
 void Problem::fill_stats() const {
@@ -1140,6 +1251,7 @@ void Problem::resolve_stats() const {
     if (!stats_pending_) return;
     check_hip(hipEventSynchronize(done_event_), "hipEventSynchronize(step)");
     stats_pending_ = false;
+    if (resident_step_) check_resident();
     for (int k = 0; k < ninst_; ++k)
         if (host_states_[k].status == kRunning)
             throw std::runtime_error("PCG: a fixed-iteration solve did not end within its enqueued rounds");

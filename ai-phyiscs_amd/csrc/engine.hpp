@@ -18,6 +18,7 @@
 
 #include "cloth_device.hpp"
 #include "cloth_kernels.hpp"
+#include "pcg_resident.hpp"
 #include "topology.hpp"
 #include "warmstart.hpp"
 
@@ -297,6 +298,17 @@ public:
         destroy_graph();
     }
 
+    // The whole solve in one launch (pcg_resident.hpp), for problems it fits:
+    // -1 where it fits, 0 never, 2 where it fits but with a start-up wait of
+    // no length, so that an instance's first workgroup solves it alone (for
+    // tests).  Results are the same bits.
+    void set_resident_solve(int mode) {
+        if (mode != -1 && mode != 0 && mode != 2) throw std::invalid_argument("resident solve: -1, 0 or 2");
+        res_mode_ = mode;
+        destroy_graph();
+    }
+    bool resident() const { return res_mode_ != 0 && res_.variant != kResidentNone; }
+
     const LaunchConfig& launch_config() const { return cfg_; }
     void set_launch_config(const LaunchConfig& c);
     // Pick the fastest launch shapes for this problem (no-op for small
@@ -320,6 +332,15 @@ private:
     // fills stats_.
     void resolve_stats() const;
     void destroy_graph();
+    // Plans the resident solve for the current storage; cols: the matrix's
+    // columns on the host.
+    void make_resident(const std::vector<int>& cols);
+    // Assembly and the resident solve, which ends with finalize; no host wait.
+    void launch_resident(float dt, const DevExt& ext, hipStream_t s);
+    void check_resident() const;
+    void train_after_solve(bool ws_on, hipStream_t s);
+    // Fills the statistics of a step whose solver states the host has.
+    void end_step(hipStream_t s);
     void warm_start_stage(float dt, const DevExt& ext, hipStream_t s);
     void push_history(hipStream_t s);
     void reset_history() { hist_n_ = 0; }
@@ -367,6 +388,18 @@ private:
     DeviceArray<float> rhs_, r_, z_, ap_, p0_, p1_;
     DeviceArray<double> x_, partials_;
     DeviceArray<int> gactive_;  // batches: 1 per group of a running instance
+
+    // resident solve
+    mutable int res_mode_ = -1;
+    bool resident_step_ = false;  // the enqueued step's solve is a resident one
+    ResidentView res_{};
+    DeviceArray<ResidentWg> res_wgs_;
+    DeviceArray<uint16_t> res_loc_;
+    DeviceArray<int> res_halo_;
+    DeviceArray<uint8_t> res_exported_;
+    DeviceArray<unsigned long long> res_zx_, res_slots_, res_ticket_;
+    DeviceArray<double> res_solo_;
+    DeviceArray<ResidentSync> res_sync_;
 
     InstState* host_states_ = nullptr;  // pinned
     mutable std::vector<SolveStats> stats_;

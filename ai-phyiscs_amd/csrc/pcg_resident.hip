@@ -1,0 +1,947 @@
+// SPDX-License-Identifier: Apache-2.0
+//
+// The PCG solve of one instance in one launch.
+//
+// One lane owns one row for the whole solve: its blocks, its Jacobi inverse,
+// r, z, p and the FP64 iterate stay in registers, and the directions that its
+// neighbours gather stay in LDS.  Nothing of the matrix is read again between
+// iterations.  What an iteration has to send through memory is z of the rows
+// that other workgroups gather (24 bytes a row) and one partial sum per
+// workgroup and inner product; both travel as 8-byte words that carry a tag
+// beside their payload, so a reader knows a word has arrived from the word
+// itself and no fence (a write-back of an XCD's whole L2) is needed.  An iteration is bound by the
+// two dependent sums over the instance's workgroups, not by bandwidth.
+//
+// Measured on MI355X, a step of 50 iterations (the streaming kernels before):
+// 21 x 21 drape 181 us (850), 64 x 64 298 us (953), 300 x 300 drape 740 us
+// (1494); a 256 x 256 cloth converged in 97 iterations 640 us (1876); 512
+// uneven cloths to convergence 12.7 ms (37.1).
+//
+// Sums, updates and the scalar step are those of the streaming kernels in the
+// same order, so the results are the same bits.
+
+#include <hip/hip_runtime.h>
+
+#include <functional>
+#include <mutex>
+#include <stdexcept>
+
+#include "pcg_device.hpp"
+#include "pcg_resident.hpp"
+
+namespace chysx_amd {
+
+[[noreturn]] void throw_hip(hipError_t err, const char* what);
+
+namespace {
+
+typedef unsigned long long u64;
+
+constexpr int kKindSigma = 0, kKindUpdate = 1, kKindTrue = 3;
+constexpr int kExchangePolls = 1 << 22;  // several seconds: a workgroup of the instance is lost
+constexpr int kMaxGroups = 256;
+
+__device__ __forceinline__ u64 agent_load(const u64* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void agent_store(u64* p, u64 v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Keep a value from being known across the loop of the iterations: what is
+// derived from it (addresses, unpacked offsets, masks) is then formed where it
+// is used instead of being held in registers for the whole solve.
+__device__ __forceinline__ int fresh(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+__device__ __forceinline__ u64 tagged(unsigned tag, unsigned v) { return (u64(tag) << 32) | v; }
+
+// Sum over the 64 lanes, in every lane: the exchanges of the xor butterfly
+// 32, 16, .., 1 by register moves.  Below a row of 16 a rotation by n reaches
+// a lane that holds the same sum as the lane n away by xor.
+template <int CTRL>
+__device__ __forceinline__ double add_rotated(double a) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(a), CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(a), CTRL, 0xf, 0xf, false);
+    return a + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double wave_sum(double a) {
+    const unsigned l0 = unsigned(__double2loint(a)), h0 = unsigned(__double2hiint(a));
+    const auto l = __builtin_amdgcn_permlane32_swap(l0, l0, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(h0, h0, false, false);
+    a = __hiloint2double(int(h[0]), int(l[0])) + __hiloint2double(int(h[1]), int(l[1]));
+    const unsigned l1 = unsigned(__double2loint(a)), h1 = unsigned(__double2hiint(a));
+    const auto m = __builtin_amdgcn_permlane16_swap(l1, l1, false, false);
+    const auto n = __builtin_amdgcn_permlane16_swap(h1, h1, false, false);
+    a = __hiloint2double(int(n[0]), int(m[0])) + __hiloint2double(int(n[1]), int(m[1]));
+    a = add_rotated<0x128>(a);
+    a = add_rotated<0x124>(a);
+    a = add_rotated<0x122>(a);
+    return add_rotated<0x121>(a);
+}
+
+// Scratch of the sums.  wave: each wave's sums, in one set per kind of sum (a
+// set is written again only after another sum's barrier); group: the group
+// sums of a many-workgroup instance.
+template <int NW>
+struct SumShared {
+    double wave[3][3][kGroupSlices];
+    double top[3][3][kGroupSlices];
+    double group[3 * (NW == 16 ? kMaxGroups : kResidentPieces * kMaxGroups / 2 + 128)];
+    int failed;
+};
+
+// What the sums need to know of the instance.
+struct Cluster {
+    int size;      // workgroups
+    int ngroups;   // groups that hold rows
+    int nslices;   // slices that hold rows
+    int group0;    // first group of the instance
+    int total;     // groups of the problem
+    int group, piece;
+    int waves;     // of this workgroup that hold rows
+    int copy;      // the copy of the sums that this workgroup reads
+    u64* slots;
+};
+
+// A sum's words: the low halves of a copy's groups, then the high halves.
+// Every workgroup reads all groups' words, so they are kept in several copies
+// for different readers: in one copy, 256 workgroups wait at a few memory
+// channels.
+__device__ __forceinline__ u64* slot_of(const Cluster& C, int kind, int piece, int copy, int group) {
+    return C.slots + ((kind * kResidentPieces + piece) * kResidentCopies + copy) * 2 * C.total + C.group0 + group;
+}
+__device__ __forceinline__ void slot_store(const Cluster& C, u64* w, unsigned tag, double d) {
+    agent_store(w, tagged(tag, unsigned(__double2loint(d))));
+    agent_store(w + C.total, tagged(tag, unsigned(__double2hiint(d))));
+}
+__device__ __forceinline__ double slot_wait(const Cluster& C, const u64* w, unsigned tag, int& failed) {
+    u64 a, b;
+    int n = 0;
+#pragma nounroll
+    do {
+        a = agent_load(w);
+        b = agent_load(w + C.total);
+    } while ((unsigned(a >> 32) != tag || unsigned(b >> 32) != tag) && ++n < kExchangePolls);
+    if (n >= kExchangePolls) failed = 1;
+    return __hiloint2double(int(unsigned(b)), int(unsigned(a)));
+}
+
+// Sums v[0 .. N) over the instance's rows; every thread gets the totals.  The
+// order is the streaming kernels': the lanes of a wave by a butterfly, the 16
+// waves of a group in order, then the groups, either as a 1024-thread workgroup
+// adds them (group t in thread t, butterfly, the waves in order) or, with
+// wave_order, as one wavefront does (lane l adds groups l, l + 64, ..., butterfly).
+// `meanwhile` runs between this workgroup's contribution and the wait for the
+// others'.  SET: the kind's set of LDS scratch.
+template <int NW, int N, int SET, class F>
+__device__ __forceinline__ bool cluster_sum(const Cluster& C, SumShared<NW>& sh, double (&v)[N], int kind,
+                                            unsigned tag, bool wave_order, double (&out)[N], F&& meanwhile) {
+    const int tid = fresh(threadIdx.x), wave = tid >> 6, lane = tid & 63;
+#pragma unroll
+    for (int j = 0; j < N; ++j) v[j] = wave_sum(v[j]);
+    if (lane == 0) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) sh.wave[SET][j][wave] = v[j];
+    }
+    __syncthreads();
+    // the group's waves in order (absent ones add zero), 8 loads in flight
+    auto in_order = [&](int j) {
+        double t = 0.0;
+#pragma unroll
+        for (int w0 = 0; w0 < NW; w0 += 8) {
+            if (w0 < C.waves) {
+                double q[8];
+#pragma unroll
+                for (int w = 0; w < 8; ++w) q[w] = sh.wave[SET][j][w0 + w];
+#pragma unroll
+                for (int w = 0; w < 8; ++w) t += q[w];
+            }
+        }
+        return t;
+    };
+    if (C.size == 1) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) out[j] = uniform_double(in_order(j));
+        meanwhile();
+        return true;
+    }
+    if (NW == 16 || C.piece == 0) {
+        const int j = tid / kResidentCopies;
+        if (j < N)
+            slot_store(C, slot_of(C, kind + j, 0, tid & (kResidentCopies - 1), C.group), tag, in_order(j));
+    } else {
+        const int w = tid / kResidentCopies, j = w >> 3;
+        if (j < N)
+            slot_store(C, slot_of(C, kind + j, 1 + (w & 7), tid & (kResidentCopies - 1), C.group), tag,
+                       sh.wave[SET][j][w & 7]);
+    }
+    int failed = 0;
+    if constexpr (NW == 16) {
+        double t[N];
+#pragma unroll
+        for (int j = 0; j < N; ++j) t[j] = 0.0;
+        if (tid < C.ngroups) {
+#pragma unroll
+            for (int j = 0; j < N; ++j) t[j] += slot_wait(C, slot_of(C, kind + j, 0, C.copy, tid), tag, failed);
+        }
+        meanwhile();
+        if (wave_order) {
+            if (tid < C.ngroups) {
+#pragma unroll
+                for (int j = 0; j < N; ++j) sh.group[j * kMaxGroups + tid] = t[j];
+            }
+        } else if (wave < kMaxGroups / 64) {
+#pragma unroll
+            for (int j = 0; j < N; ++j) t[j] = wave_sum(t[j]);
+            if (lane == 0) {
+#pragma unroll
+                for (int j = 0; j < N; ++j) sh.top[SET][j][wave] = t[j];
+            }
+        }
+        if (failed) sh.failed = 1;
+        __syncthreads();
+        if (wave_order) {
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                double a = 0.0;
+#pragma nounroll
+                for (int q = lane; q < C.ngroups; q += 64) a += sh.group[j * kMaxGroups + q];
+                out[j] = wave_sum(a);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                double a = 0.0;
+#pragma unroll
+                for (int w = 0; w < kMaxGroups / 64; ++w) a += sh.top[SET][j][w];
+                out[j] = a;
+            }
+        }
+    } else {
+        // A group's first half is one value, its second half's waves are 8:
+        // a few values a thread, all loaded before any is looked at.
+        const int per = kResidentPieces * C.ngroups;
+        constexpr int kBatch = N == 1 ? 3 : 5;
+#pragma nounroll
+        for (int q0 = tid; q0 < N * per; q0 += kBatch * NW * 64) {
+            const u64* w[kBatch];
+            bool there[kBatch];
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) {
+                const int q = q0 + u * NW * 64, j = q / per, pg = q - j * per, p = pg / C.ngroups, g = pg - p * C.ngroups;
+                there[u] = q < N * per && (p == 0 || C.nslices > 16 * g + 8 + (p - 1));
+                w[u] = there[u] ? slot_of(C, kind + j, p, C.copy, g) : slot_of(C, kind, 0, C.copy, 0);
+            }
+            u64 a[kBatch], b[kBatch];
+            int n = 0;
+            bool late;
+#pragma nounroll
+            do {
+                late = false;
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) {
+                    a[u] = agent_load(w[u]);
+                    b[u] = agent_load(w[u] + C.total);
+                }
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u)
+                    late = late || unsigned(a[u] >> 32) != tag || unsigned(b[u] >> 32) != tag;
+            } while (late && ++n < kExchangePolls);
+            if (late) failed = 1;
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) {
+                const int q = q0 + u * NW * 64;
+                if (q < N * per)
+                    sh.group[q] = there[u] ? __hiloint2double(int(unsigned(b[u])), int(unsigned(a[u]))) : 0.0;
+            }
+        }
+        meanwhile();
+        if (failed) sh.failed = 1;
+        __syncthreads();
+        // wave (2 j + c) sums value j of the groups 64 c .. 64 c + 63
+        if (wave < 2 * N) {
+            const int j = wave >> 1, g = (wave & 1) * 64 + lane;
+            double t = 0.0;
+            if (g < C.ngroups) {
+                double q[kResidentPieces];
+#pragma unroll
+                for (int p = 0; p < kResidentPieces; ++p) q[p] = sh.group[j * per + p * C.ngroups + g];
+#pragma unroll
+                for (int p = 0; p < kResidentPieces; ++p) t += q[p];
+            }
+            if (wave_order) sh.group[3 * kResidentPieces * (kMaxGroups / 2) + wave * 64 + lane] = t;
+            else t = wave_sum(t);
+            if (lane == 0) sh.top[SET][j][wave & 1] = t;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            if (wave_order) {
+                const double* q = sh.group + 3 * kResidentPieces * (kMaxGroups / 2) + j * 128 + lane;
+                out[j] = wave_sum((0.0 + q[0]) + q[64]);
+            } else {
+                out[j] = (0.0 + sh.top[SET][j][0]) + sh.top[SET][j][1];
+            }
+        }
+        // the next sum writes sh.group again only after its own barrier
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j) out[j] = uniform_double(out[j]);
+    return uniform_int(sh.failed) == 0;
+}
+
+// The instance's workgroups agree that they run: all of them have started, so
+// every wait that follows ends.  If they have not met within R.meet_polls (the
+// device's compute units are held by waiting workgroups of another process),
+// one of them solves the instance alone and the others leave.
+enum Meeting : int { kMeetRun = 0, kMeetLeave = 1, kMeetAlone = 2 };
+__device__ int meet(ResidentSync* S, int cluster, int polls) {
+    const u64 a = __hip_atomic_fetch_add(&S->arrived, u64(1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const u64 run = 2 * (a / u64(cluster) + 1);
+    if ((a + 1) % u64(cluster) == 0) {
+        u64 old = agent_load(&S->decision);
+        if (old < run)
+            __hip_atomic_compare_exchange_strong(&S->decision, &old, run, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT);
+    }
+#pragma nounroll
+    for (int n = 0; n < polls; ++n) {
+        const u64 d = agent_load(&S->decision);
+        if (d >= run) return d == run ? kMeetRun : kMeetLeave;
+        __builtin_amdgcn_s_sleep(2);
+    }
+    u64 old = agent_load(&S->decision);
+    if (old < run && __hip_atomic_compare_exchange_strong(&S->decision, &old, run + 1, __ATOMIC_RELAXED,
+                                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        return kMeetAlone;
+    return old == run ? kMeetRun : kMeetLeave;
+}
+
+// Blocks of one row in the order the streaming kernel adds them, and where
+// their columns' vectors lie in LDS.
+template <bool PK, int MAXW>
+struct Blocks {
+    float m[MAXW][PK ? 6 : 9];
+    unsigned at[(MAXW + 1) / 2];  // two 16-bit byte offsets each
+};
+
+template <bool PK, int MAXW>
+__device__ __forceinline__ void load_blocks(const DevMatrix& A, const uint16_t* __restrict__ loc, int row, int sb,
+                                            int w, unsigned zero, Blocks<PK, MAXW>& B) {
+    const int lane = row & 63;
+#pragma unroll
+    for (int k = 0; k < (MAXW + 1) / 2; ++k) B.at[k] = zero * 0x10001u;
+#pragma unroll
+    for (int k = 0; k < MAXW; ++k) {
+#pragma unroll
+        for (int q = 0; q < (PK ? 6 : 9); ++q) B.m[k][q] = 0.0f;
+        if (k < w) {  // wave-uniform
+            const int kk = (PK || A.sym) ? sym_order(k, w) : k;
+            const size_t e = size_t(sb + kk) * 64 + lane;
+            const int c = A.col[e];
+            if (c >= 0) {
+                if (PK) {
+                    const float* b = A.val + (c < row ? val_offset(A.mir[e], 6) : size_t(sb + kk) * 6 * 64 + lane);
+#pragma unroll
+                    for (int q = 0; q < 6; ++q) B.m[k][q] = b[q * 64];
+                } else {
+                    float m[9];
+                    load_block(A, A.val + size_t(sb + kk) * 9 * 64 + lane, A.mir + e, c, row, m);
+#pragma unroll
+                    for (int q = 0; q < 9; ++q) B.m[k][PK ? 0 : q] = m[q];
+                }
+            }
+            B.at[k >> 1] = (k & 1) ? (B.at[k >> 1] & 0xFFFFu) | (unsigned(loc[e]) << 16)
+                                   : (B.at[k >> 1] & 0xFFFF0000u) | unsigned(loc[e]);
+        }
+        // one entry's loads at a time: issued together, those of every entry
+        // would need more registers than the blocks themselves
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// The solve of one instance by one workgroup, its vectors in global memory:
+// the way out when the instance's workgroups cannot all run at once.
+template <int NW>
+__device__ __forceinline__ void solve_alone(const ResidentView& R, const LaunchGeom& g, const DevMatrix& A, const DevVectors& v,
+                            const DevExt& e, const DevMesh& m, const InstParams& pr, InstState& S, float dt,
+                            int given_r, SumShared<NW>& sh) {
+    const int tid = threadIdx.x, wave = uniform_int(tid >> 6), lane = tid & 63;
+    const int s0 = S.slice0, ns = S.nslices, ng = (ns + kGroupSlices - 1) / kGroupSlices;
+    float* p = v.p0;
+    // sums of the slices' values in R.solo[slot * nslices + slice], in the streaming kernels' order
+    auto total = [&](int slot, bool wave_order) {
+        double* part = R.solo + size_t(slot) * g.nslices + s0;
+        __syncthreads();
+        for (int q = tid; q < ng; q += NW * 64) {
+            double t = 0.0;
+            for (int w = 0; w < kGroupSlices; ++w) t += 16 * q + w < ns ? part[16 * q + w] : 0.0;
+            sh.group[q] = t;
+        }
+        __syncthreads();
+        double a = 0.0;
+        for (int q0 = 0; q0 < ng; q0 += 64) {
+            const double t = q0 + lane < ng ? sh.group[q0 + lane] : 0.0;
+            if (wave_order) a += t;
+            else a += wave_sum(t);
+        }
+        const double out = wave_order ? wave_sum(a) : a;
+        __syncthreads();
+        return out;
+    };
+    auto put = [&](int slot, int s, double val) {
+        val = wave_sum(val);
+        if (lane == 0) R.solo[size_t(slot) * g.nslices + s] = val;
+    };
+    // true residual of every row; r, z = p = M^-1 r unless it is only reported
+    auto residual = [&](bool report, bool from_r) {
+        for (int q = wave; q < ns; q += NW) {
+            const int s = s0 + q, row = s * 64 + lane;
+            const SliceDesc sd = g.slices[s];
+            double a = 0.0, b = 0.0, c = 0.0;
+            if (lane < sd.nvalid) {
+                F3 rf, bf;
+                if (from_r) {
+                    rf = ld3(v.r, row);
+                    bf = ld3(v.rhs, row);
+                    a = fma3d(0.0, rf.x, rf.y, rf.z, rf.x, rf.y, rf.z);
+                } else {
+                    double r[3];
+                    bf = true_residual<false>(A, v, s, lane, sd.nlower, r);
+                    rf = f3(float(r[0]), float(r[1]), float(r[2]));
+                    a = fma3d(0.0, r[0], r[1], r[2], r[0], r[1], r[2]);
+                }
+                b = fma3d(0.0, bf.x, bf.y, bf.z, bf.x, bf.y, bf.z);
+                if (!report) {
+                    const F3 zf = minv_mul(A, s, lane, rf);
+                    st3(v.r, row, rf);
+                    st3(v.z, row, zf);
+                    st3(p, row, zf);
+                    c = fma3d(0.0, rf.x, rf.y, rf.z, zf.x, zf.y, zf.z);
+                }
+            }
+            put(0, s, a);
+            put(1, s, b);
+            put(2, s, c);
+        }
+    };
+    residual(false, given_r != 0);
+    {
+        const double rr = total(0, true), bb = total(1, true), rz = total(2, true);
+        pcg_begin(S, pr, rr, bb, rz);
+    }
+    while (S.status == kRunning) {
+        if (S.mode == kModeCheck) {
+            residual(false, false);
+            const double rr = total(0, false), rz = total(2, false);
+            pcg_advance(S, pr, AdvanceSums{rz, rr});
+            continue;
+        }
+        const float beta = float(S.beta);
+        // the owed term of a deferred update needs the direction it belongs to
+        for (int q = wave; q < ns; q += NW) {
+            const int row = (s0 + q) * 64 + lane;
+            if (lane < g.slices[s0 + q].nvalid) {
+                const F3 old = ld3(p, row);
+                st3(v.p1, row, old);
+                st3(p, row, dir3(ld3(v.z, row), old, beta));
+            }
+        }
+        __syncthreads();
+        for (int q = wave; q < ns; q += NW) {
+            const int s = s0 + q, row = s * 64 + lane;
+            double a = 0.0;
+            if (lane < g.slices[s].nvalid) {
+                const int sb = A.slice_ptr[s], w = A.slice_ptr[s + 1] - sb;
+                float d[9];
+                load_diag(A, s, lane, d);
+                const F3 pi = ld3(p, row);
+                F3 y = f3(fma3(0.0f, d[0], d[1], d[2], pi), fma3(0.0f, d[3], d[4], d[5], pi),
+                          fma3(0.0f, d[6], d[7], d[8], pi));
+                for (int k = 0; k < w; ++k) {
+                    const int kk = A.sym ? sym_order(k, w) : k;
+                    const size_t en = size_t(sb + kk) * 64 + lane;
+                    const int c = A.col[en];
+                    if (c < 0) continue;
+                    load_block(A, A.val + size_t(sb + kk) * A.bs * 64 + lane, A.mir + en, c, row, d);
+                    const F3 pj = ld3(p, c);
+                    y = f3(fma3(y.x, d[0], d[1], d[2], pj), fma3(y.y, d[3], d[4], d[5], pj),
+                           fma3(y.z, d[6], d[7], d[8], pj));
+                }
+                st3(v.ap, row, y);
+                a = fma3d(0.0, double(pi.x), double(pi.y), double(pi.z), y.x, y.y, y.z);
+            }
+            put(0, s, a);
+        }
+        const double sig = total(0, false);
+        const double alpha = (sig > kGuard || sig < -kGuard) ? S.rho / sig : 0.0;
+        for (int q = wave; q < ns; q += NW) {
+            const int s = s0 + q, row = s * 64 + lane;
+            double a = 0.0, b = 0.0;
+            if (lane < g.slices[s].nvalid) {
+                const F3 pi = ld3(p, row), pp = ld3(v.p1, row);
+                double* x = v.x + 3 * row;
+                if (S.pend) {
+                    x[0] = x_two(x[0], S.alpha_pend, pp.x, alpha, pi.x);
+                    x[1] = x_two(x[1], S.alpha_pend, pp.y, alpha, pi.y);
+                    x[2] = x_two(x[2], S.alpha_pend, pp.z, alpha, pi.z);
+                } else if (!S.defer) {
+                    x[0] = fma(alpha, double(pi.x), x[0]);
+                    x[1] = fma(alpha, double(pi.y), x[1]);
+                    x[2] = fma(alpha, double(pi.z), x[2]);
+                }
+                const float* mv = A.minv + (size_t)s * 6 * 64 + lane;
+                const float mi[6] = {mv[0], mv[64], mv[128], mv[192], mv[256], mv[320]};
+                const F3 r = r_update(ld3(v.r, row), ld3(v.ap, row), float(alpha));
+                const F3 z = z_update(mi, r);
+                st3(v.r, row, r);
+                st3(v.z, row, z);
+                a = dot3d(r, z);
+                b = dot3d(r, r);
+            }
+            put(0, s, a);
+            put(1, s, b);
+        }
+        const double rz = total(0, false), rr = total(1, false);
+        S.sigma = sig;
+        S.alpha = alpha;
+        pcg_advance(S, pr, AdvanceSums{rz, rr});
+        if (S.status == kRunning && S.mode == kModeFlush) {
+            for (int q = wave; q < ns; q += NW) {
+                const int row = (s0 + q) * 64 + lane;
+                if (lane < g.slices[s0 + q].nvalid) {
+                    const F3 pi = ld3(p, row);
+                    double* x = v.x + 3 * row;
+                    x[0] = fma(S.alpha_pend, double(pi.x), x[0]);
+                    x[1] = fma(S.alpha_pend, double(pi.y), x[1]);
+                    x[2] = fma(S.alpha_pend, double(pi.z), x[2]);
+                }
+            }
+            __syncthreads();
+            pcg_advance(S, pr, AdvanceSums{0.0, 0.0});
+        }
+    }
+    if (S.status == kStopped) {
+        residual(true, false);
+        S.rr = total(0, true);
+        S.relres = sqrt(S.rr / S.bb);
+    }
+    for (int q = wave; q < ns; q += NW) {
+        const SliceDesc sd = g.slices[s0 + q];
+        const int row = (s0 + q) * 64 + lane;
+        if (lane < sd.nvalid)
+            finalize_row(e, pr, dt, m.pin_inc_off, m.pin_inc, m.pin_tgt, row, sd.part0 + lane, v.x[3 * row],
+                         v.x[3 * row + 1], v.x[3 * row + 2]);
+    }
+}
+
+// Every field in scalar registers: all threads hold the same state.
+__device__ __forceinline__ void uniform_state(InstState& S) {
+    S.rho = uniform_double(S.rho);
+    S.bb = uniform_double(S.bb);
+    S.rr = uniform_double(S.rr);
+    S.beta = uniform_double(S.beta);
+    S.relres = uniform_double(S.relres);
+    S.alpha = uniform_double(S.alpha);
+    S.alpha_pend = uniform_double(S.alpha_pend);
+    S.status = uniform_int(S.status);
+    S.mode = uniform_int(S.mode);
+    S.iters = uniform_int(S.iters);
+    S.restarts = uniform_int(S.restarts);
+    S.parity = uniform_int(S.parity);
+    S.pend = uniform_int(S.pend);
+    S.defer = uniform_int(S.defer);
+}
+
+// The outcome of a solve; what was set at build time stays.
+__device__ __forceinline__ void store_state(const InstState& S, InstState& mem, InstState& host) {
+    for (InstState* q : {&mem, &host}) {
+        q->rho = S.rho;
+        q->bb = S.bb;
+        q->rr = S.rr;
+        q->beta = S.beta;
+        q->relres = S.relres;
+        q->status = S.status;
+        q->mode = S.mode;
+        q->iters = S.iters;
+        q->restarts = S.restarts;
+        q->parity = S.parity;
+        q->alpha_pend = S.alpha_pend;
+        q->pend = S.pend;
+        q->defer = S.defer;
+        q->owed = 0;
+    }
+}
+
+template <bool PK, int MAXW, int NW>
+__global__ __launch_bounds__(64 * NW) void pcg_resident_kernel(ResidentView R, LaunchGeom g, DevMatrix A,
+                                                               DevVectors v, DevExt e, DevMesh m,
+                                                               InstState* __restrict__ st,
+                                                               InstState* __restrict__ host_st,
+                                                               const InstParams* __restrict__ params, float dt,
+                                                               int given_r) {
+    extern __shared__ __align__(16) float lds[];
+    __shared__ SumShared<NW> sh;
+    __shared__ int shared_int[2];
+    const int tid = threadIdx.x, wave = uniform_int(tid >> 6), lane = tid & 63;
+    const int threads = int(blockDim.x);
+    int wgi = blockIdx.x;
+    if (R.max_cluster > 1) {
+        // Workgroups take their places in the order they start, so those of
+        // the instances before theirs have all started and free their compute
+        // units: a batch whose workgroups do not all fit at once goes through.
+        if (tid == 0)
+            shared_int[0] = int(__hip_atomic_fetch_add(R.ticket, u64(1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) %
+                                u64(R.nwg));
+        __syncthreads();
+        wgi = __builtin_amdgcn_readfirstlane(shared_int[0]);
+    }
+    const ResidentWg W = R.wgs[wgi];
+    const InstParams& pr = params[W.inst];
+    InstState& mem = st[W.inst];
+    // absent waves add nothing
+    for (int q = tid; q < 3 * 3 * kGroupSlices; q += threads) (&sh.wave[0][0][0])[q] = 0.0;
+    if (tid == 0) sh.failed = 0;
+    Cluster C;
+    C.size = W.cluster;
+    C.nslices = mem.nslices;
+    C.ngroups = (C.nslices + kGroupSlices - 1) / kGroupSlices;
+    C.group0 = mem.group0;
+    C.total = g.ngroups;
+    C.group = W.group;
+    C.piece = W.piece;
+    C.waves = W.nslices;
+    C.copy = (wgi - W.first) & (kResidentCopies - 1);
+    C.slots = R.slots;
+    unsigned tag = 0;
+    if (W.cluster > 1) {
+        tag = R.sync[W.inst].epoch;
+        if (tid == 0) shared_int[1] = meet(R.sync + W.inst, W.cluster, R.meet_polls);
+    } else if (tid == 0) {
+        shared_int[1] = kMeetRun;
+    }
+    __syncthreads();
+    const int met = __builtin_amdgcn_readfirstlane(shared_int[1]);
+    if (met == kMeetLeave) return;
+    if (met == kMeetAlone) {
+        InstState S = mem;
+        solve_alone<NW>(R, g, A, v, e, m, pr, S, dt, given_r, sh);
+        if (tid == 0) store_state(S, mem, host_st[W.inst]);
+        return;
+    }
+    InstState S{};  // the fields that the solve works with
+    S.parity = mem.parity;
+
+    const int s = __builtin_amdgcn_readfirstlane(W.slice0 + wave);
+    const bool live = wave < W.nslices;
+    SliceDesc sd{};
+    if (live) sd = g.slices[s];
+    const bool valid = lane < sd.nvalid;
+    const int row = s * 64 + lane;
+    const int own = W.nslices * 64;  // LDS rows: own, halo, zero
+    float* mine = lds + 3 * (wave * 64 + lane);
+    float* zin = lds + 3 * R.lds_rows;  // z of the halo rows as received
+    if (tid < 3) lds[3 * (own + W.nhalo) + tid] = 0.0f;
+    const bool sends = valid && R.exported[row] != 0;
+    auto nothing = [] {};
+    // z of a row in two words, x with half of y and z with the other half, each
+    // with the low 16 bits of the tag: a row's words are written once for every
+    // tag that sends, so an old word never has the tag waited for.
+    auto send_z = [&](F3 z, unsigned t) {
+        if (sends) {
+            u64* w = R.zx + fresh(row);
+            const unsigned y = __float_as_uint(z.y);
+            agent_store(w, tagged((t << 16) | (y & 0xFFFFu), __float_as_uint(z.x)));
+            agent_store(w + R.rows, tagged((t << 16) | (y >> 16), __float_as_uint(z.z)));
+        }
+    };
+    // The halo rows' z with tag t, into zin.  The last threads start, since
+    // the first ones wait for the sums.
+    auto receive_z = [&](unsigned t) {
+#pragma nounroll
+        for (int h = threads - 1 - fresh(tid); h < W.nhalo; h += threads) {
+            const u64* w = R.zx + R.halo[W.halo0 + h];
+            u64 a, b;
+            int n = 0;
+#pragma nounroll
+            do {
+                a = agent_load(w);
+                b = agent_load(w + R.rows);
+            } while ((((unsigned(a >> 32) ^ (t << 16)) | (unsigned(b >> 32) ^ (t << 16))) > 0xFFFFu) &&
+                     ++n < kExchangePolls);
+            if (n >= kExchangePolls) sh.failed = 1;
+            zin[3 * h] = __uint_as_float(unsigned(a));
+            zin[3 * h + 1] = __uint_as_float((unsigned(a >> 32) & 0xFFFFu) | (unsigned(b >> 32) << 16));
+            zin[3 * h + 2] = __uint_as_float(unsigned(b));
+        }
+    };
+
+    // The iterate and the direction that an owed term belongs to are touched
+    // every other iteration: they lie in LDS, where they cost no registers.
+    double* xl = reinterpret_cast<double*>(lds + R.lds_x) + 3 * tid;
+    float* pl = lds + R.lds_x + 6 * threads + 3 * tid;
+    F3 r = f3(0.0f, 0.0f, 0.0f), z = r, p = r;
+    if (valid) {
+        xl[0] = v.x[3 * row];
+        xl[1] = v.x[3 * row + 1];
+        xl[2] = v.x[3 * row + 2];
+    }
+    // The iterate goes to memory, for the residual's gathers and the next
+    // step's guess.  Every wave's stores have arrived before its workgroup
+    // contributes to the sum that all wait for.
+    auto publish_x = [&] {
+        if (valid) {
+            double* xo = v.x + 3 * fresh(row);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) __hip_atomic_store(xo + c, xl[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_s_waitcnt(0);
+        double none[1] = {0.0}, got[1];
+        ++tag;
+        return cluster_sum<NW, 1, 0>(C, sh, none, kKindSigma, tag, false, got, nothing);
+    };
+    // Each round begins with a true residual: the start's, the check of a
+    // solve whose recursive residual has passed the test, or the report of a
+    // stopped one.
+    enum Phase : int { kBegin, kCheck, kReport };
+    int phase = kBegin;
+    bool met_all = true;  // no wait ran out (left as a flag: a return from here would make the loops' exits divergent)
+    for (;;) {
+        {
+            double part[3] = {0.0, 0.0, 0.0}, sum[3];
+            if (valid) {
+                const int ln = fresh(lane);
+                if (phase == kBegin && given_r) {  // pcg_start_given_r_kernel
+                    r = ld3(v.r, s * 64 + ln);
+                    const F3 bf = ld3(v.rhs, s * 64 + ln);
+                    part[0] = fma3d(0.0, r.x, r.y, r.z, r.x, r.y, r.z);
+                    part[1] = fma3d(0.0, bf.x, bf.y, bf.z, bf.x, bf.y, bf.z);
+                } else {
+                    double rd[3];
+                    const F3 bf = true_residual<true>(A, v, s, ln, sd.nlower, rd);
+                    r = f3(float(rd[0]), float(rd[1]), float(rd[2]));
+                    part[0] = fma3d(0.0, rd[0], rd[1], rd[2], rd[0], rd[1], rd[2]);
+                    part[1] = fma3d(0.0, bf.x, bf.y, bf.z, bf.x, bf.y, bf.z);
+                }
+                z = minv_mul(A, s, ln, r);
+                part[2] = fma3d(0.0, r.x, r.y, r.z, z.x, z.y, z.z);
+            }
+            ++tag;
+            send_z(z, tag);
+            met_all = cluster_sum<NW, 3, 2>(C, sh, part, kKindTrue, tag, phase != kCheck, sum, [&] { receive_z(tag); });
+            if (!met_all) break;
+            if (phase == kBegin) {
+                pcg_begin(S, pr, sum[0], sum[1], sum[2]);
+            } else if (phase == kCheck) {
+                pcg_advance(S, pr, AdvanceSums{sum[2], sum[0]});
+            } else {
+                S.rr = sum[0];
+                S.relres = sqrt(sum[0] / S.bb);
+            }
+            uniform_state(S);
+            if (phase == kReport || S.status == kConverged) break;
+            if (S.status == kStopped) {  // no iterations left after a failed check
+                met_all = publish_x();
+                if (!met_all) break;
+                phase = kReport;
+                continue;
+            }
+        }
+        // Everything is set on every path, so that none of it stays live
+        // through the next round's residual.
+        Blocks<PK, MAXW> B;
+        float dg[PK ? 6 : 9], mi[6];
+#pragma unroll
+        for (int q = 0; q < (PK ? 6 : 9); ++q) dg[q] = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 6; ++q) mi[q] = 0.0f;
+        const int sb = live ? A.slice_ptr[s] : 0;
+        const int w = live ? A.slice_ptr[s + 1] - sb : 0;
+        load_blocks<PK, MAXW>(A, R.loc, fresh(row), sb, w, 12u * unsigned(own + W.nhalo), B);
+        if (live) {
+            const float* dp = A.diag + (size_t)s * (PK ? 6 : 9) * 64 + fresh(lane);
+#pragma unroll
+            for (int q = 0; q < (PK ? 6 : 9); ++q) dg[q] = dp[q * 64];
+            const float* mv = A.minv + (size_t)s * 6 * 64 + fresh(lane);
+#pragma unroll
+            for (int q = 0; q < 6; ++q) mi[q] = mv[q * 64];
+        }
+        bool first = true;  // a (re)start: p_prev = z, beta = 0
+        while (S.status == kRunning && S.mode == kModeIter) {
+            const float beta = float(S.beta);
+            if (valid) {
+                p = dir3(z, first ? z : p, beta);
+                mine[0] = p.x;
+                mine[1] = p.y;
+                mine[2] = p.z;
+            }
+#pragma nounroll
+            for (int h = threads - 1 - fresh(tid); h < W.nhalo; h += threads) {
+                float* ph = lds + 3 * (own + h);
+                const F3 zh = ld3(zin, h);
+                const F3 d = dir3(zh, first ? zh : f3(ph[0], ph[1], ph[2]), beta);
+                ph[0] = d.x;
+                ph[1] = d.y;
+                ph[2] = d.z;
+            }
+            first = false;
+            __syncthreads();
+            F3 ap = f3(0.0f, 0.0f, 0.0f);
+            double sg[1] = {0.0}, sig[1];
+            if (valid) {
+                if (PK) {
+                    ap.x = fma3(0.0f, dg[0], dg[1], dg[2], p);
+                    ap.y = fma3(0.0f, dg[1], dg[3], dg[4], p);
+                    ap.z = fma3(0.0f, dg[2], dg[4], dg[5], p);
+                } else {
+                    ap.x = fma3(0.0f, dg[0], dg[1], dg[2], p);
+                    ap.y = fma3(0.0f, dg[3], dg[4], dg[5], p);
+                    ap.z = fma3(0.0f, dg[PK ? 0 : 6], dg[PK ? 0 : 7], dg[PK ? 0 : 8], p);
+                }
+                // entries past the slice's width are zero blocks on the zero
+                // row: no branch parts the gathers
+#pragma unroll
+                for (int k = 0; k < MAXW; ++k) {
+                    const unsigned at = unsigned(fresh(int(B.at[k >> 1])));
+                    const float* q = reinterpret_cast<const float*>(reinterpret_cast<const char*>(lds) +
+                                                                    ((k & 1) ? at >> 16 : at & 0xFFFFu));
+                    const F3 pj = f3(q[0], q[1], q[2]);
+                    const float* b = B.m[k];
+                    if (PK) {
+                        ap.x = fma3(ap.x, b[0], b[1], b[2], pj);
+                        ap.y = fma3(ap.y, b[1], b[3], b[4], pj);
+                        ap.z = fma3(ap.z, b[2], b[4], b[5], pj);
+                    } else {
+                        ap.x = fma3(ap.x, b[0], b[1], b[2], pj);
+                        ap.y = fma3(ap.y, b[3], b[4], b[5], pj);
+                        ap.z = fma3(ap.z, b[PK ? 0 : 6], b[PK ? 0 : 7], b[PK ? 0 : 8], pj);
+                    }
+                }
+                sg[0] = fma3d(0.0, double(p.x), double(p.y), double(p.z), ap.x, ap.y, ap.z);
+            }
+            ++tag;
+            met_all = cluster_sum<NW, 1, 0>(C, sh, sg, kKindSigma, tag, false, sig, nothing);
+            if (!met_all) break;
+            const double alpha = (sig[0] > kGuard || sig[0] < -kGuard) ? S.rho / sig[0] : 0.0;
+            double part[2] = {0.0, 0.0}, sum[2];
+            ++tag;
+            if (valid) {
+                r = r_update(r, ap, float(alpha));
+                z = z_update(mi, r);
+                send_z(z, tag);
+                part[0] = dot3d(r, z);
+                part[1] = dot3d(r, r);
+                if (S.pend) {  // the owed term and this one
+                    xl[0] = x_two(xl[0], S.alpha_pend, pl[0], alpha, p.x);
+                    xl[1] = x_two(xl[1], S.alpha_pend, pl[1], alpha, p.y);
+                    xl[2] = x_two(xl[2], S.alpha_pend, pl[2], alpha, p.z);
+                } else if (S.defer) {
+                    pl[0] = p.x;
+                    pl[1] = p.y;
+                    pl[2] = p.z;
+                } else {
+                    xl[0] = fma(alpha, double(p.x), xl[0]);
+                    xl[1] = fma(alpha, double(p.y), xl[1]);
+                    xl[2] = fma(alpha, double(p.z), xl[2]);
+                }
+            }
+            met_all = cluster_sum<NW, 2, 1>(C, sh, part, kKindUpdate, tag, false, sum, [&] { receive_z(tag); });
+            if (!met_all) break;
+            S.alpha = alpha;
+            pcg_advance(S, pr, AdvanceSums{sum[0], sum[1]});
+        }
+        if (met_all && S.status == kRunning && S.mode == kModeFlush) {
+            if (valid) {
+                xl[0] = fma(S.alpha_pend, double(p.x), xl[0]);
+                xl[1] = fma(S.alpha_pend, double(p.y), xl[1]);
+                xl[2] = fma(S.alpha_pend, double(p.z), xl[2]);
+            }
+            pcg_advance(S, pr, AdvanceSums{0.0, 0.0});
+            uniform_state(S);
+        }
+        if (!met_all) break;
+        met_all = publish_x();
+        if (!met_all) break;
+        phase = S.status == kStopped ? kReport : kCheck;
+    }
+    if (!met_all) {
+        if (tid == 0) {
+            mem.status = kResidentTimedOut;
+            host_st[W.inst].status = kResidentTimedOut;
+        }
+        return;
+    }
+    if (valid) {
+        const int own_row = fresh(row);  // this lane's own words of v.x
+        finalize_row(e, pr, dt, m.pin_inc_off, m.pin_inc, m.pin_tgt, own_row, sd.part0 + lane, v.x[3 * own_row],
+                     v.x[3 * own_row + 1], v.x[3 * own_row + 2]);
+    }
+    if (wgi == W.first && tid == 0) {
+        store_state(S, mem, host_st[W.inst]);
+        if (W.cluster > 1) R.sync[W.inst].epoch = tag;
+    }
+}
+
+// Launches whose instances span more than kFreeCluster workgroups run one
+// after the other on a device, whatever their streams: two that each hold part
+// of the compute units while they wait for the rest would not meet.  Smaller
+// ones never hold enough of them (at most 32 hardware queues with 7 waiting
+// workgroups each, of 256 compute units) and stay free.
+constexpr int kFreeCluster = 8;
+constexpr int kMaxDevices = 64;
+struct Gate {
+    std::mutex lock;
+    hipEvent_t last = nullptr;  // the latest gated launch
+    hipStream_t stream = nullptr;
+};
+Gate& gate_of_device() {
+    static Gate gates[kMaxDevices];
+    int dev = 0;
+    const hipError_t err = hipGetDevice(&dev);
+    if (err != hipSuccess) throw_hip(err, "hipGetDevice");
+    if (dev < 0 || dev >= kMaxDevices) throw std::runtime_error("chysx: device index out of range");
+    return gates[dev];
+}
+
+}  // namespace
+
+void with_resident_gate(int max_cluster, hipStream_t s, const std::function<void()>& enqueue) {
+    if (max_cluster <= kFreeCluster) {
+        enqueue();
+        return;
+    }
+    auto check = [](hipError_t err, const char* what) {
+        if (err != hipSuccess) throw_hip(err, what);
+    };
+    Gate& G = gate_of_device();
+    const std::lock_guard<std::mutex> hold(G.lock);
+    if (!G.last) check(hipEventCreateWithFlags(&G.last, hipEventDisableTiming), "hipEventCreate(resident solve)");
+    else if (G.stream != s) check(hipStreamWaitEvent(s, G.last, 0), "hipStreamWaitEvent(resident solve)");
+    enqueue();
+    check(hipEventRecord(G.last, s), "hipEventRecord(resident solve)");
+    G.stream = s;
+}
+
+void launch_pcg_resident(const ResidentView& R, const LaunchGeom& g, const DevMatrix& A, const DevVectors& v,
+                         const DevExt& e, const DevMesh& m, InstState* st, InstState* host_st,
+                         const InstParams* params, float dt, int start_given_r, hipStream_t s) {
+    if (R.nwg <= 0) return;
+    if (g.ngroups * kGroupSlices != g.nslices) throw std::invalid_argument("resident solve: whole 16-slice groups");
+    if ((R.variant == kResidentC) != (A.bs == 9) || (R.max_cluster > 1 && R.block_waves != R.waves))
+        throw std::invalid_argument("resident solve: the plan was made for another storage");
+    const int block = 64 * R.block_waves;
+#define CHYSX_RESIDENT(PK, MAXW, NW)                                                                             \
+    pcg_resident_kernel<PK, MAXW, NW><<<R.nwg, block, R.lds_bytes, s>>>(R, g, A, v, e, m, st, host_st, params, dt, \
+                                                                        start_given_r)
+    if (R.variant == kResidentA) CHYSX_RESIDENT(true, kResidentWidthA, 16);
+    else if (R.variant == kResidentB) CHYSX_RESIDENT(true, kResidentWidthB, 8);
+    else if (R.variant == kResidentC) CHYSX_RESIDENT(false, kResidentWidthC, 8);
+    else throw std::invalid_argument("resident solve: no plan");
+#undef CHYSX_RESIDENT
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) throw_hip(err, "pcg_resident_kernel");
+}
+
+}  // namespace chysx_amd

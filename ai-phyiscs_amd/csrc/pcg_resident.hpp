@@ -1,0 +1,125 @@
+// SPDX-License-Identifier: Apache-2.0
+//
+// The whole PCG solve of an instance as one launch: host plan and device view.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+#include <functional>
+#include <vector>
+
+#include "cloth_kernels.hpp"
+
+namespace chysx_amd {
+
+// One workgroup of the resident solve: up to `waves` consecutive slices of
+// one instance.  A 16-wave workgroup owns one 16-slice group; 8-wave ones own
+// half a group each (piece 0 or 1).  An instance's workgroups are consecutive.
+struct ResidentWg {
+    int inst;
+    int slice0;   // first slice
+    int nslices;  // slices holding rows
+    int group;    // group within the instance
+    int piece;
+    int halo0;    // first entry of its halo list
+    int nhalo;    // rows of other workgroups that its rows couple to
+    int cluster;  // workgroups of the instance
+    int first;    // the instance's first workgroup
+};
+
+// The three kernels, by what a lane's row takes of the registers: up to
+// kResidentWidthA packed blocks (a grid's six, 36 registers) leave room for 16
+// waves a compute unit at 128 registers; wider rows (96) and 9-float blocks
+// (126) take 8 waves at 256.  One row a lane: what is left of a lane's
+// registers would not hold a second row, and a problem that needs more
+// workgroups than the device has compute units streams its matrix instead
+// (512 x 512 is the largest square cloth here, 362 x 362 with bending).
+enum ResidentVariant : int { kResidentNone = 0, kResidentA = 1, kResidentB = 2, kResidentC = 3 };
+constexpr int kResidentWidthA = 6;   // packed
+constexpr int kResidentWidthB = 16;  // packed
+constexpr int kResidentWidthC = 14;  // 9 floats
+
+constexpr int kResidentMaxWgs = 256;       // workgroups of an instance
+constexpr int kResidentStaticLds = 36864;  // LDS of the kernels beside the dynamic part
+constexpr int kResidentMeetPolls = 400000;  // about half a second
+
+struct ResidentPlan {
+    int variant = kResidentNone;
+    int waves = 0;
+    int max_nslices = 0;        // widest workgroup
+    int max_cluster = 0;
+    int lds_rows = 0;           // own and halo rows of the largest workgroup, and the zero row
+    int max_halo = 0;
+    std::vector<ResidentWg> wgs;
+    std::vector<uint16_t> loc;  // per matrix entry: byte offset of its column's vector in LDS
+    std::vector<int> halo;      // row indices, ascending per workgroup
+    std::vector<uint8_t> exported;  // per row: 1 when another workgroup needs it
+};
+
+// One instance's rows for the plan.
+struct ResidentInstance {
+    int slice0, nslices;  // slices holding rows
+};
+
+// Plan for rows of `bs`-float blocks in the wave-sliced ELL layout (columns in
+// row space, -1 for padding).  variant kResidentNone: the problem stays with
+// the kernels that stream the matrix (a row is too wide, an instance needs
+// more than `max_wgs` workgroups, or a workgroup's own and halo rows do not
+// fit in max_lds bytes).
+ResidentPlan plan_resident(const std::vector<ResidentInstance>& insts, const std::vector<int>& slice_ptr,
+                           const std::vector<int>& cols, int bs, int max_wgs, int max_lds);
+
+// Start-up agreement of an instance's workgroups, kept in device memory across
+// launches (all zero at first).
+struct ResidentSync {
+    unsigned long long arrived;   // workgroups started, over all launches
+    unsigned long long decision;  // 2 L: launch L (1, 2, ...) runs; 2 L + 1: its workgroups did not meet in time
+    unsigned epoch;               // last tag used in the exchange words
+    unsigned pad;
+};
+
+struct ResidentView {
+    int variant, waves, block_waves, nwg, lds_rows, lds_x, lds_bytes, max_cluster;
+    const ResidentWg* wgs;
+    const uint16_t* loc;
+    const int* halo;
+    const uint8_t* exported;
+    unsigned long long* zx;     // 2 words a row (all first words, then all second ones): z of the exported rows
+    int rows;                   // padded rows of the problem
+    unsigned long long* slots;  // partial sums: kinds x pieces x copies x 2 halves x groups words
+    double* solo;               // 3 per slice: partial sums of an instance solved by one workgroup
+    ResidentSync* sync;         // per instance
+    unsigned long long* ticket;
+    int meet_polls;             // bound of the start-up wait, in polls of about a microsecond
+};
+constexpr int kResidentKinds = 6;   // 0: p . Ap; 1, 2: r . z, |r|^2; 3 .. 5: start, check and report sums
+constexpr int kResidentPieces = 9;  // a group's sum, or its first half's and the waves of its second
+// LDS of a workgroup, in floats: 3 a row for the own, halo and zero rows, 3 a
+// halo row as received, then (8-byte aligned) 9 a lane for the iterate and a
+// direction.
+inline int resident_lds_x(int lds_rows, int max_halo) { return (3 * (lds_rows + max_halo) + 1) & ~1; }
+inline int resident_lds_bytes(int lds_rows, int max_halo, int block_waves) {
+    return 4 * (resident_lds_x(lds_rows, max_halo) + 9 * 64 * block_waves);
+}
+constexpr int kResidentCopies = 8;  // copies of the sums, for different readers
+inline size_t resident_slot_words(int ngroups) {
+    return size_t(kResidentKinds) * kResidentPieces * kResidentCopies * 2 * size_t(ngroups);
+}
+
+// Status a solve is left with when a wait of the exchange ran out (reported
+// as an error by the host; it takes a lost workgroup).
+constexpr int kResidentTimedOut = 4;
+
+// Start residual, iterations, true-residual checks, report residual and
+// finalize of every instance, from the assembled system.  host_st: the solver
+// states in pinned host memory.  start_given_r: the start residual is in v.r.
+void launch_pcg_resident(const ResidentView& R, const LaunchGeom& g, const DevMatrix& A, const DevVectors& v,
+                         const DevExt& e, const DevMesh& m, InstState* st, InstState* host_st,
+                         const InstParams* params, float dt, int start_given_r, hipStream_t s);
+
+// Runs `enqueue`, which puts a resident solve on stream s, in turn with the
+// device's other ones when its instances span many workgroups.
+void with_resident_gate(int max_cluster, hipStream_t s, const std::function<void()>& enqueue);
+
+}  // namespace chysx_amd

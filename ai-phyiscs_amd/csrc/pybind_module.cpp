@@ -419,6 +419,10 @@ PYBIND11_MODULE(_chysx_native, m) {
                  return out;
              })
         .def(
+            "set_resident_solve",
+            [](Sim& s, int mode) { check(chysx_cloth_set_resident_solve(s.p(), mode)); }, py::arg("mode"),
+            "-1: the whole solve in one launch where the problem fits it; 0: never (speed only, the same bits).")
+        .def(
             "set_pin_projection", [](Sim& s, bool on) { check(chysx_cloth_set_pin_projection(s.p(), on ? 1 : 0)); },
             py::arg("on"),
             "True: pins are constraints (each pinned particle ends every step exactly at its target); False "
@@ -664,6 +668,9 @@ PYBIND11_MODULE(_chysx_native, m) {
         .def(
             "set_blocking_step", [](Batch& b, bool on) { check(chysx_batch_set_blocking_step(b.h, on ? 1 : 0)); },
             py::arg("on"))
+        .def(
+            "set_resident_solve",
+            [](Batch& b, int mode) { check(chysx_batch_set_resident_solve(b.h, mode)); }, py::arg("mode"))
         .def(
             "set_pin_projection",
             [](Batch& b, bool on) { check(chysx_batch_set_pin_projection(b.h, on ? 1 : 0)); }, py::arg("on"))

@@ -193,6 +193,11 @@ int chysx_cloth_set_external_force_active(chysx_cloth* sim, int on);
  * the free rows, its own row becomes the identity), so it ends every step
  * exactly at its target; the pin stiffness is unused.  Default 0 (penalty). */
 int chysx_cloth_set_pin_projection(chysx_cloth* sim, int on);
+/* Extension: where the solve runs.  -1 (default): in one launch that keeps the
+ * matrix in registers, for cloths it fits (up to 256 workgroups); 0: always in
+ * the kernels that stream the matrix; 2: as -1, with a start-up wait of no
+ * length, after which one workgroup solves alone (tests).  Same bits. */
+int chysx_cloth_set_resident_solve(chysx_cloth* sim, int mode);
 int chysx_cloth_pin_projection(const chysx_cloth* sim, int* out);
 /* Per-element stiffness (one value per spring in edge order / per triangle). */
 int chysx_cloth_set_spring_stiffnesses(chysx_cloth* sim, const float* k, int n);
@@ -253,6 +258,8 @@ int chysx_batch_set_blocking_step(chysx_batch* b, int on);
 int chysx_batch_set_split_advance(chysx_batch* b, int mode);
 /* Pin projection (as chysx_cloth_set_pin_projection) for every cloth of the batch. */
 int chysx_batch_set_pin_projection(chysx_batch* b, int on);
+/* Where the solves run (as chysx_cloth_set_resident_solve). */
+int chysx_batch_set_resident_solve(chysx_batch* b, int mode);
 int chysx_batch_stats(const chysx_batch* b, int index, int* iters, int* restarts, int* status, double* relres);
 /* Number of cloths added to the batch. */
 int chysx_batch_num_cloths(const chysx_batch* b, int* n);
