@@ -65,6 +65,8 @@ template class DeviceArray<uint16_t>;
 template class DeviceArray<uint8_t>;
 template class DeviceArray<unsigned long long>;
 template class DeviceArray<ResidentSync>;
+template class DeviceArray<SweepWg>;
+template class DeviceArray<unsigned>;
 
 // ---------------------------------------------------------------------------
 // Rest data
@@ -495,6 +497,7 @@ void Problem::build(const std::vector<const Instance*>& insts) {
 
 void Problem::make_resident(const std::vector<int>& cols) {
     res_ = ResidentView{};
+    sweep_ = SweepView{};
     int dev = 0, cus = 0, lds = 0;
     check_hip(hipGetDevice(&dev), "hipGetDevice");
     check_hip(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute(CUs)");
@@ -507,7 +510,10 @@ void Problem::make_resident(const std::vector<int>& cols) {
     }
     const ResidentPlan P = plan_resident(insts, slice_ptr_h_, cols, block_floats(), std::min(cus, kResidentMaxWgs),
                                          lds - kResidentStaticLds);
-    if (P.variant == kResidentNone || P.wgs.empty()) return;
+    if (P.variant == kResidentNone || P.wgs.empty()) {
+        make_sweep(cols, std::min(cus, kResidentMaxWgs), lds);
+        return;
+    }
     hipStream_t s = nullptr;
     res_wgs_.assign(P.wgs.data(), P.wgs.size(), s);
     res_loc_.assign(P.loc.data(), P.loc.size(), s);
@@ -544,6 +550,60 @@ void Problem::make_resident(const std::vector<int>& cols) {
     res_.variant = P.variant;
 }
 
+void Problem::make_sweep(const std::vector<int>& cols, int max_wgs, int lds) {
+    if (ninst_ != 1 || block_floats() != 6) return;
+    const int used = (inst_n_[0] + kSlice - 1) / kSlice, ngroups = (used + kGroupSlices - 1) / kGroupSlices;
+    if (ngroups <= max_wgs || ngroups > max_wgs * kSweepMaxGroups) return;
+    std::vector<int> nlower(slices_h_.size());
+    for (size_t k = 0; k < nlower.size(); ++k) nlower[k] = slices_h_[k].nlower;
+    const SweepPlan P = plan_sweep(used, slice_ptr_h_, cols, mir_h_, nlower, max_wgs, lds - kSweepStaticLds);
+    if (P.groups == 0) return;
+    hipStream_t s = nullptr;
+    sweep_wgs_.assign(P.wgs.data(), P.wgs.size(), s);
+    sweep_packed_.assign(P.packed.data(), P.packed.size(), s);
+    sweep_zeros_.resize(6 * kSlice);
+    sweep_zeros_.zero(s);
+    res_halo_.assign(P.halo.data(), P.halo.size(), s);
+    res_exported_.assign(P.exported.data(), P.exported.size(), s);
+    res_zx_.resize(size_t(n_pad_) * 2);
+    res_slots_.resize(sweep_slot_words(ngroups));
+    res_solo_.resize(size_t(nslices()) * 3);
+    res_sync_.resize(1);
+    res_zx_.zero(s);
+    res_slots_.zero(s);
+    res_sync_.zero(s);
+    check_hip(hipStreamSynchronize(s), "hipStreamSynchronize(sweep plan)");
+    sweep_.nwg = int(P.wgs.size());
+    sweep_.ngroups = ngroups;
+    sweep_.lds_rows = P.lds_rows;
+    sweep_.max_halo = P.max_halo;
+    sweep_.rows = n_pad_;
+    sweep_.wgs = sweep_wgs_.data();
+    sweep_.packed = sweep_packed_.data();
+    sweep_.zeros = sweep_zeros_.data();
+    sweep_.halo = res_halo_.data();
+    sweep_.exported = res_exported_.data();
+    sweep_.zx = res_zx_.data();
+    sweep_.slots = res_slots_.data();
+    sweep_.solo = res_solo_.data();
+    sweep_.sync = res_sync_.data();
+    sweep_.meet_polls = kResidentMeetPolls;
+    sweep_.groups = P.groups;
+}
+
+void Problem::launch_sweep(hipStream_t s) {
+    SweepView R = sweep_;
+    if (res_mode_ == 2) R.meet_polls = 0;
+    const LaunchGeom g = geom();
+    with_resident_gate(R.nwg, s, [&] { launch_pcg_sweep(R, g, matrix(), vectors(), state_.data(), params_.data(), s); });
+    bool checks = false;
+    for (const InstParams& q : params_h_) checks = checks || q.tol2 > 0.0;
+    if (!checks) return;
+    launch_pcg_spmv(g, matrix(), vectors(), state_.data(), nullptr, nullptr, cfg_.spmv_unroll, s, cfg_.spmv_branch_free,
+                    cfg_.spmv_symmetric);
+    launch_pcg_advance(state_.data(), params_.data(), partials_.data(), ninst_, g.ngroups, s, g.gactive);
+}
+
 void Problem::launch_resident(float dt, const DevExt& ext, hipStream_t s) {
     ResidentView R = res_;
     if (res_mode_ == 2) R.meet_polls = 0;
@@ -555,9 +615,10 @@ void Problem::launch_resident(float dt, const DevExt& ext, hipStream_t s) {
     });
 }
 
-void Problem::check_resident() const {
+void Problem::check_resident(bool running) const {
     for (int k = 0; k < ninst_; ++k)
-        if (host_states_[k].status != kConverged && host_states_[k].status != kStopped) {
+        if (host_states_[k].status != kConverged && host_states_[k].status != kStopped &&
+            !(running && host_states_[k].status == kRunning)) {
             res_mode_ = 0;  // the exchange words are in no known state
             throw std::runtime_error("PCG: a solve lost one of its workgroups");
         }
@@ -1112,7 +1173,7 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
     proj_ran_ = false;
     start_r_ready_ = false;
     const bool ws_on = ws_mode_ != kWarmPrevious || ws_train_;
-    if (resident()) {
+    if (resident() || sweeps()) {
         // the solve is launched directly, not as a graph, so a capture is refused here
         hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
         check_hip(hipStreamIsCapturing(s, &capturing), "hipStreamIsCapturing");
@@ -1134,16 +1195,17 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
         // long fixed solves replay the chunk graphs instead, so a graph never
         // holds more than kStepGraphMaxChunks chunks
         const int chunks = std::max(1, (fixed_iters + 2 + kChunkIters - 1) / kChunkIters);
-        resident_step_ = resident();
-        if (resident_step_) {
+        resident_step_ = resident() || sweeps();
+        if (resident()) {
             launch_assemble(dt, ext, s);
             launch_resident(dt, ext, s);
-        } else if (chunks <= kStepGraphMaxChunks) {
+        } else if (!sweeps() && chunks <= kStepGraphMaxChunks) {
             launch_fixed_step_graph(dt, ext, chunks, s);
         } else {
             launch_assemble(dt, ext, s);
             launch_pcg_start(s);
-            launch_pcg_chunks(s, chunks);
+            if (sweeps()) launch_sweep(s);
+            else launch_pcg_chunks(s, chunks);
             launch_pcg_residual(geom(), matrix(), vectors(), state_.data(), 1, s);
             launch_pcg_reduce(state_.data(), params_.data(), partials_.data(), ninst_, geom().ngroups, kPhaseFinal,
                               s);
@@ -1177,8 +1239,10 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
     int chunks = std::max(1, (last_iters_ + 2 + kChunkIters - 1) / kChunkIters);
     int guard = 0;
     for (;;) {
-        launch_pcg_chunks(s, chunks);
+        if (sweeps()) launch_sweep(s);
+        else launch_pcg_chunks(s, chunks);
         read_states(s);
+        if (sweeps()) check_resident(true);
         if (all_done()) break;
         chunks = 1;
         if (++guard > (1 << 22)) throw std::runtime_error("PCG did not terminate");

@@ -19,6 +19,7 @@
 #include "cloth_device.hpp"
 #include "cloth_kernels.hpp"
 #include "pcg_resident.hpp"
+#include "pcg_sweep.hpp"
 #include "topology.hpp"
 #include "warmstart.hpp"
 
@@ -298,7 +299,8 @@ public:
         destroy_graph();
     }
 
-    // The whole solve in one launch (pcg_resident.hpp), for problems it fits:
+    // The solve, or a large cloth's iterations, in one launch (pcg_resident.hpp,
+    // pcg_sweep.hpp), for problems that fit:
     // -1 where it fits, 0 never, 2 where it fits but with a start-up wait of
     // no length, so that an instance's first workgroup solves it alone (for
     // tests).  Results are the same bits.
@@ -308,6 +310,9 @@ public:
         destroy_graph();
     }
     bool resident() const { return res_mode_ != 0 && res_.variant != kResidentNone; }
+    // A single cloth too large for that whose vectors fit the chip: its
+    // iterations run in one launch (pcg_sweep.hpp).
+    bool sweeps() const { return res_mode_ != 0 && sweep_.groups != 0; }
 
     const LaunchConfig& launch_config() const { return cfg_; }
     void set_launch_config(const LaunchConfig& c);
@@ -335,9 +340,14 @@ private:
     // Plans the resident solve for the current storage; cols: the matrix's
     // columns on the host.
     void make_resident(const std::vector<int>& cols);
+    void make_sweep(const std::vector<int>& cols, int max_wgs, int lds);
+    // The iterations of a started solve until its next true-residual check,
+    // and that check; no host wait.
+    void launch_sweep(hipStream_t s);
     // Assembly and the resident solve, which ends with finalize; no host wait.
     void launch_resident(float dt, const DevExt& ext, hipStream_t s);
-    void check_resident() const;
+    // Throws when a solve lost a workgroup (or, unless `running`, has not ended).
+    void check_resident(bool running = false) const;
     void train_after_solve(bool ws_on, hipStream_t s);
     // Fills the statistics of a step whose solver states the host has.
     void end_step(hipStream_t s);
@@ -400,6 +410,10 @@ private:
     DeviceArray<unsigned long long> res_zx_, res_slots_, res_ticket_;
     DeviceArray<double> res_solo_;
     DeviceArray<ResidentSync> res_sync_;
+    SweepView sweep_{};
+    DeviceArray<SweepWg> sweep_wgs_;
+    DeviceArray<unsigned> sweep_packed_;
+    DeviceArray<float> sweep_zeros_;
 
     InstState* host_states_ = nullptr;  // pinned
     mutable std::vector<SolveStats> stats_;
