@@ -68,7 +68,13 @@ struct Cluster {
     int waves;     // of this workgroup that hold rows
     int copy;      // the copy of the sums that this workgroup reads
     u64* slots;
+    int pause, pause_z;  // before the first look, see exchange_pause
 };
+
+__device__ __forceinline__ void pause(int n) {
+#pragma nounroll
+    for (; n > 0; --n) __builtin_amdgcn_s_sleep(1);
+}
 
 // A sum's words: the low halves of a copy's groups, then the high halves.
 // Every workgroup reads all groups' words, so they are kept in several copies

@@ -13,9 +13,9 @@
 // two dependent sums over the instance's workgroups, not by bandwidth.
 //
 // Measured on MI355X, a step of 50 iterations (the streaming kernels before):
-// 21 x 21 drape 181 us (850), 64 x 64 298 us (953), 300 x 300 drape 740 us
-// (1494); a 256 x 256 cloth converged in 97 iterations 640 us (1876); 512
-// uneven cloths to convergence 12.7 ms (37.1).
+// 21 x 21 drape 182 us (850), 64 x 64 294 us (953), 300 x 300 drape 615 us
+// (1494); a 256 x 256 cloth converged in 97 iterations 595 us (1876); 512
+// uneven cloths to convergence 12.4 ms (37.1).
 //
 // Sums, updates and the scalar step are those of the streaming kernels in the
 // same order, so the results are the same bits.
@@ -95,7 +95,9 @@ __device__ __forceinline__ bool cluster_sum(const Cluster& C, SumShared<NW>& sh,
                        sh.wave[SET][j][w & 7]);
     }
     int failed = 0;
+    pause(N == 1 ? C.pause : C.pause_z);
     if constexpr (NW == 16) {
+        meanwhile();
         double t[N];
 #pragma unroll
         for (int j = 0; j < N; ++j) t[j] = 0.0;
@@ -103,7 +105,6 @@ __device__ __forceinline__ bool cluster_sum(const Cluster& C, SumShared<NW>& sh,
 #pragma unroll
             for (int j = 0; j < N; ++j) t[j] += slot_wait(C, slot_of(C, kind + j, 0, C.copy, tid), tag, failed);
         }
-        meanwhile();
         if (wave_order) {
             if (tid < C.ngroups) {
 #pragma unroll
@@ -137,6 +138,10 @@ __device__ __forceinline__ bool cluster_sum(const Cluster& C, SumShared<NW>& sh,
             }
         }
     } else {
+        // few workgroups: the sums come soon after z (20 half groups: 2.83 ms,
+        // and 2.95 ms with z first; 176: 637 us, and 610)
+        const bool z_first = C.pause >= 18;
+        if (z_first) meanwhile();
         // A group's first half is one value, its second half's waves are 8:
         // a few values a thread, all loaded before any is looked at.
         const int per = kResidentPieces * C.ngroups;
@@ -174,7 +179,7 @@ __device__ __forceinline__ bool cluster_sum(const Cluster& C, SumShared<NW>& sh,
                     sh.group[q] = there[u] ? __hiloint2double(int(unsigned(b[u])), int(unsigned(a[u]))) : 0.0;
             }
         }
-        meanwhile();
+        if (!z_first) meanwhile();
         if (failed) sh.failed = 1;
         __syncthreads();
         // wave (2 j + c) sums value j of the groups 64 c .. 64 c + 63
@@ -324,6 +329,8 @@ __global__ __launch_bounds__(64 * NW) void pcg_resident_kernel(ResidentView R, L
     C.waves = W.nslices;
     C.copy = (wgi - W.first) & (kResidentCopies - 1);
     C.slots = R.slots;
+    C.pause = W.pause;
+    C.pause_z = W.pause_z;
     unsigned tag = 0;
     if (W.cluster > 1) {
         tag = R.sync[W.inst].epoch;

@@ -5,6 +5,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <functional>
 #include <vector>
@@ -26,6 +28,8 @@ struct ResidentWg {
     int nhalo;    // rows of other workgroups that its rows couple to
     int cluster;  // workgroups of the instance
     int first;    // the instance's first workgroup
+    int pause;    // before it looks for a sum of one value, and for the
+    int pause_z;  // neighbours' z with an update's sums: s_sleep units
 };
 
 // The three kernels, by what a lane's row takes of the registers: up to
@@ -56,6 +60,27 @@ struct ResidentPlan {
     std::vector<int> halo;      // row indices, ascending per workgroup
     std::vector<uint8_t> exported;  // per row: 1 when another workgroup needs it
 };
+
+// How long a workgroup waits, in s_sleep units of 64 cycles, before it first
+// looks for the sums of `wgs` workgroups.  The words need some 2600 cycles to
+// arrive, and those of the slowest workgroup come the later the more there
+// are; a look before that takes a round trip of 1500 cycles itself and,
+// together with every other workgroup's, holds up the words looked for.  None
+// up to 24 workgroups (12 units cost 2% at 4 and 1% at 20), then 12, and 6 more
+// with each doubling beyond 32: within 3% of the best of 0 to 32 units at 32 to
+// 256 workgroups.  An iteration without and with it: 6.0 and 5.4 us at 64
+// workgroups, 9.0 and 6.4 at 157, 10.0 and 8.4 at 256; 12.3 and 10.3 us at 176
+// half-group workgroups.
+inline int exchange_pause(int wgs) { return wgs <= 24 ? 0 : std::max(12, int(std::lround(6.0 * std::log2(wgs / 8.0)))); }
+// The same before the neighbours' z, which is sent ahead of an update's sums:
+// 6 units less.  `wide`: even the wave that waits for the sums has halo rows
+// to receive, and their wait is most of the pause.  From 480 x 480 on 6 units
+// are best (512 x 512: 8.5 us an iteration against 8.9 with 18), up to
+// 430 x 430 the difference of 6 is (8.2 us with 18 units, 9.1 with 6).
+inline int exchange_pause_z(int wgs, bool wide) {
+    const int p = exchange_pause(wgs) - 6;
+    return p <= 0 ? 0 : wide ? std::min(p, 6) : p;
+}
 
 // One instance's rows for the plan.
 struct ResidentInstance {

@@ -11,10 +11,10 @@
 // also pay two more launches.  z of the boundary rows and the sums travel as in
 // the resident solve.
 //
-// At 1024 x 1024 an iteration takes 32 us against 53 us (76.9 K cycles: 31 to
-// 36 K in the products, 16 to 23 K for p . Ap with 5 to 12 K of it waiting for
-// the slowest workgroup, 17 K for the update's sums with the iterate under
-// them), and solves to 1e-6 take 11.2 ms where they took 18.7 ms.  The products
+// At 1024 x 1024 an iteration takes 31 us against 53 us (about 75 K cycles: 31
+// to 36 K in the products, 15 to 22 K for p . Ap with 5 to 12 K of it waiting
+// for the slowest workgroup, 17 K for the update's sums with the iterate under
+// them), and three steps solved to 1e-6 take 10.9 ms where they took 18.7 ms.  The products
 // read 4.5 TB/s from the Infinity Cache; with 8 waves a compute unit more loads
 // in flight would need registers that the vectors hold.  Fewer, larger pieces
 // (2 groups at 512 x 512 on half the units) lose to the resident solve, and
@@ -131,6 +131,7 @@ __device__ __forceinline__ bool sweep_sum(const SweepView& R, const SweepWg& W, 
             agent_store(w + R.ngroups, tagged(tag, unsigned(__double2hiint(t))));
         }
     }
+    if (N == 1) pause(R.pause);
     meanwhile();
     const int copy = int(blockIdx.x) & (kResidentCopies - 1);
     double t[N][2];

@@ -59,6 +59,7 @@ struct SweepView {
     double* solo;               // 3 per slice
     ResidentSync* sync;
     int meet_polls;
+    int pause;  // before the look for p . Ap; the update's sums wait behind the iterate and need none
 };
 inline size_t sweep_slot_words(int ngroups) { return size_t(kSweepKinds) * kResidentCopies * 2 * size_t(ngroups); }
 inline int sweep_lds_bytes(int groups, int lds_rows, int max_halo) {
