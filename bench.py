@@ -495,7 +495,7 @@ def cpu_baseline(args, s, g, cpu_state):
 def reference_mode(args, scene, make_sim):
     """The reference's own stopping rule on the same cloth: a fixed 50 PCG
     iterations per step, no convergence test (pcg_solver.cu:542-592).  Each
-    step is one captured graph launched without a host wait; the window is
+    step is enqueued without a host wait; the window is
     timed from the first launch to the stream's end."""
     import torch
     g = make_sim(scene, tol=0.0, max_iter=50)

@@ -153,9 +153,11 @@ int chysx_cloth_pcg_iterations(const chysx_cloth* sim, int* out);
  * after its graph launch (pcg_solver.cu:882-894); pos / vel are updated when
  * the stream reaches that point.  The solve statistics wait for it.  With a
  * tolerance (chysx_cloth_set_pcg_tolerance > 0) or a warm-start stage the
- * step synchronises `stream` once per poll of the solver state (after the
- * iterations the previous step needed, then every 8) and returns when the
- * solve has ended, with the pos / vel update enqueued behind it on `stream`.
+ * step synchronises `stream` once per poll of the solver state (once where the
+ * whole solve is one launch, per true-residual check for one cloth up to
+ * 1024x1024, else after the iterations the previous step needed, then every 8)
+ * and returns when the solve has ended, with the pos / vel update done or
+ * enqueued behind it on `stream`.
  * Consecutive steps may use different streams: each is ordered after the
  * previous one. */
 int chysx_cloth_step(chysx_cloth* sim, float dt, uintptr_t stream);
@@ -194,7 +196,8 @@ int chysx_cloth_set_external_force_active(chysx_cloth* sim, int on);
  * exactly at its target; the pin stiffness is unused.  Default 0 (penalty). */
 int chysx_cloth_set_pin_projection(chysx_cloth* sim, int on);
 /* Extension: where the solve runs.  -1 (default): in one launch that keeps the
- * matrix in registers, for cloths it fits (up to 256 workgroups); 0: always in
+ * matrix in registers, for cloths it fits (up to 256 workgroups), or, for one
+ * regularly triangulated cloth up to 1024x1024, its vectors; 0: always in
  * the kernels that stream the matrix; 2: as -1, with a start-up wait of no
  * length, after which one workgroup solves alone (tests).  Same bits. */
 int chysx_cloth_set_resident_solve(chysx_cloth* sim, int mode);
