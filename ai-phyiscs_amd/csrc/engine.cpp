@@ -588,7 +588,7 @@ void Problem::make_sweep(const std::vector<int>& cols, int max_wgs, int lds) {
     sweep_.solo = res_solo_.data();
     sweep_.sync = res_sync_.data();
     sweep_.meet_polls = kResidentMeetPolls;
-    sweep_.pause = exchange_pause(sweep_.nwg);
+    sweep_.pause = exchange_pause(sweep_.nwg, false);
     sweep_.groups = P.groups;
 }
 

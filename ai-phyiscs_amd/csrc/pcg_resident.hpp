@@ -66,19 +66,23 @@ struct ResidentPlan {
 // arrive, and those of the slowest workgroup come the later the more there
 // are; a look before that takes a round trip of 1500 cycles itself and,
 // together with every other workgroup's, holds up the words looked for.  None
-// up to 24 workgroups (12 units cost 2% at 4 and 1% at 20), then 12, and 6 more
-// with each doubling beyond 32: within 3% of the best of 0 to 32 units at 32 to
-// 256 workgroups.  An iteration without and with it: 6.0 and 5.4 us at 64
-// workgroups, 9.0 and 6.4 at 157, 10.0 and 8.4 at 256; 12.3 and 10.3 us at 176
-// half-group workgroups.
-inline int exchange_pause(int wgs) { return wgs <= 24 ? 0 : std::max(12, int(std::lround(6.0 * std::log2(wgs / 8.0)))); }
+// up to 8 workgroups (12 units cost 2% at 4) or, of half groups, whose looks
+// take nine words a group, up to 24 (12 units cost 1% at 20); then 12 (512
+// cloths of up to 16 workgroups: 25.3 ms without and 24.8 with, 150 x 150: 5.5
+// and 5.3 us an iteration), and 6 more with each doubling beyond 32: within 3%
+// of the best of 0 to 32 units at 32 to 256 workgroups.  An iteration without
+// and with it: 6.0 and 5.4 us at 64 workgroups, 9.0 and 6.4 at 157, 10.0 and
+// 8.4 at 256; 12.3 and 10.3 us at 176 half-group workgroups.
+inline int exchange_pause(int wgs, bool halves) {
+    return wgs <= (halves ? 24 : 8) ? 0 : std::max(12, int(std::lround(6.0 * std::log2(wgs / 8.0))));
+}
 // The same before the neighbours' z, which is sent ahead of an update's sums:
 // 6 units less.  `wide`: even the wave that waits for the sums has halo rows
 // to receive, and their wait is most of the pause.  From 480 x 480 on 6 units
 // are best (512 x 512: 8.5 us an iteration against 8.9 with 18), up to
 // 430 x 430 the difference of 6 is (8.2 us with 18 units, 9.1 with 6).
-inline int exchange_pause_z(int wgs, bool wide) {
-    const int p = exchange_pause(wgs) - 6;
+inline int exchange_pause_z(int wgs, bool halves, bool wide) {
+    const int p = exchange_pause(wgs, halves) - 6;
     return p <= 0 ? 0 : wide ? std::min(p, 6) : p;
 }
 

@@ -46,7 +46,7 @@ ResidentPlan plan_resident(const std::vector<ResidentInstance>& insts, const std
             W.piece = (c * P.waves % kGroupSlices) / P.waves;
             W.cluster = cluster;
             W.first = first;
-            W.pause = exchange_pause(cluster);
+            W.pause = exchange_pause(cluster, P.waves < kGroupSlices);
             const int r0 = W.slice0 * 64, nr = W.nslices * 64;
             halo.clear();
             const size_t e0 = size_t(slice_ptr[size_t(W.slice0)]) * 64;
@@ -82,7 +82,7 @@ ResidentPlan plan_resident(const std::vector<ResidentInstance>& insts, const std
         }
     }
     if (resident_lds_bytes(P.lds_rows, P.max_halo, P.waves) > max_lds) return none;
-    for (ResidentWg& W : P.wgs) W.pause_z = exchange_pause_z(W.cluster, P.max_halo > 64 * (P.waves - 1));
+    for (ResidentWg& W : P.wgs) W.pause_z = exchange_pause_z(W.cluster, P.waves < kGroupSlices, P.max_halo > 64 * (P.waves - 1));
     return P;
 }
 
