@@ -508,8 +508,7 @@ void Problem::make_resident(const std::vector<int>& cols) {
         insts[size_t(k)].slice0 = inst_slice0_[size_t(k)];
         insts[size_t(k)].nslices = (inst_n_[size_t(k)] + kSlice - 1) / kSlice;
     }
-    const ResidentPlan P = plan_resident(insts, slice_ptr_h_, cols, block_floats(), std::min(cus, kResidentMaxWgs),
-                                         lds - kResidentStaticLds);
+    const ResidentPlan P = plan_resident(insts, slice_ptr_h_, cols, block_floats(), cus, lds - kResidentStaticLds);
     if (P.variant == kResidentNone || P.wgs.empty()) {
         make_sweep(cols, std::min(cus, kResidentMaxWgs), lds);
         return;
@@ -536,6 +535,7 @@ void Problem::make_resident(const std::vector<int>& cols) {
     res_.lds_x = resident_lds_x(P.lds_rows, P.max_halo);
     res_.lds_bytes = resident_lds_bytes(P.lds_rows, P.max_halo, res_.block_waves);
     res_.max_cluster = P.max_cluster;
+    res_.by_start = P.by_start ? 1 : 0;
     res_.wgs = res_wgs_.data();
     res_.loc = res_loc_.data();
     res_.halo = res_halo_.data();

@@ -302,10 +302,7 @@ __global__ __launch_bounds__(64 * NW) void pcg_resident_kernel(ResidentView R, L
     const int tid = threadIdx.x, wave = uniform_int(tid >> 6), lane = tid & 63;
     const int threads = int(blockDim.x);
     int wgi = blockIdx.x;
-    if (R.max_cluster > 1) {
-        // Workgroups take their places in the order they start, so those of
-        // the instances before theirs have all started and free their compute
-        // units: a batch whose workgroups do not all fit at once goes through.
+    if (R.by_start) {  // places in the order of starting (plan_resident says when)
         if (tid == 0)
             shared_int[0] = int(__hip_atomic_fetch_add(R.ticket, u64(1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) %
                                 u64(R.nwg));

@@ -53,6 +53,9 @@ struct ResidentPlan {
     int waves = 0;
     int max_nslices = 0;        // widest workgroup
     int max_cluster = 0;
+    // Workgroups take their places in the order they start, not by their
+    // number (resident_by_start).
+    bool by_start = false;
     int lds_rows = 0;           // own and halo rows of the largest workgroup, and the zero row
     int max_halo = 0;
     std::vector<ResidentWg> wgs;
@@ -60,6 +63,23 @@ struct ResidentPlan {
     std::vector<int> halo;      // row indices, ascending per workgroup
     std::vector<uint8_t> exported;  // per row: 1 when another workgroup needs it
 };
+
+// Which workgroup takes which place of a launch of `wgs` workgroups on `cus`
+// compute units.  An XCD is given every 8th workgroup, in order, and no other,
+// and a workgroup here has a compute unit to itself.
+// In the order they start (true): at most one instance has only part of its
+// workgroups running, and an XCD that is ahead takes more places than one that
+// is behind (512 uneven cloths: 24.8 ms, and 26.1 ms by number).  But the
+// waiting part of an instance must not be able to fill an XCD: the missing
+// workgroups may be bound to that XCD, and then all wait until the start-up
+// agreement gives up (two cloths of 198 workgroups: 164 ms a step on average,
+// 0.8 ms by number).
+// By number (false): an instance lies evenly over the XCDs, and the first one
+// that has not met is next in line on each of them, so it always comes to run.
+constexpr int kXcds = 8;
+inline bool resident_by_start(int wgs, int max_cluster, int cus) {
+    return max_cluster > 1 && (wgs <= cus || max_cluster <= cus / kXcds);
+}
 
 // How long a workgroup waits, in s_sleep units of 64 cycles, before it first
 // looks for the sums of `wgs` workgroups.  The words need some 2600 cycles to
@@ -92,12 +112,12 @@ struct ResidentInstance {
 };
 
 // Plan for rows of `bs`-float blocks in the wave-sliced ELL layout (columns in
-// row space, -1 for padding).  variant kResidentNone: the problem stays with
-// the kernels that stream the matrix (a row is too wide, an instance needs
-// more than `max_wgs` workgroups, or a workgroup's own and halo rows do not
-// fit in max_lds bytes).
+// row space, -1 for padding), on `cus` compute units.  variant kResidentNone:
+// the problem stays with the kernels that stream the matrix (a row is too
+// wide, an instance needs more than `cus` or kResidentMaxWgs workgroups, or a
+// workgroup's own and halo rows do not fit in max_lds bytes).
 ResidentPlan plan_resident(const std::vector<ResidentInstance>& insts, const std::vector<int>& slice_ptr,
-                           const std::vector<int>& cols, int bs, int max_wgs, int max_lds);
+                           const std::vector<int>& cols, int bs, int cus, int max_lds);
 
 // Start-up agreement of an instance's workgroups, kept in device memory across
 // launches (all zero at first).
@@ -110,6 +130,7 @@ struct ResidentSync {
 
 struct ResidentView {
     int variant, waves, block_waves, nwg, lds_rows, lds_x, lds_bytes, max_cluster;
+    int by_start;               // as ResidentPlan
     const ResidentWg* wgs;
     const uint16_t* loc;
     const int* halo;
@@ -119,7 +140,7 @@ struct ResidentView {
     unsigned long long* slots;  // partial sums: kinds x pieces x copies x 2 halves x groups words
     double* solo;               // 3 per slice: partial sums of an instance solved by one workgroup
     ResidentSync* sync;         // per instance
-    unsigned long long* ticket;
+    unsigned long long* ticket; // workgroups started, over all launches (by_start)
     int meet_polls;             // bound of the start-up wait, in polls of about a microsecond
 };
 constexpr int kResidentKinds = 6;   // 0: p . Ap; 1, 2: r . z, |r|^2; 3 .. 5: start, check and report sums

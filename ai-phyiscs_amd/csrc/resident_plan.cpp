@@ -8,8 +8,9 @@
 namespace chysx_amd {
 
 ResidentPlan plan_resident(const std::vector<ResidentInstance>& insts, const std::vector<int>& slice_ptr,
-                           const std::vector<int>& cols, int bs, int max_wgs, int max_lds) {
+                           const std::vector<int>& cols, int bs, int cus, int max_lds) {
     ResidentPlan none, P;
+    const int max_wgs = std::min(cus, kResidentMaxWgs);
     int width = 0;
     for (size_t s = 0; s + 1 < slice_ptr.size(); ++s) width = std::max(width, slice_ptr[s + 1] - slice_ptr[s]);
     if (bs == 6 && width <= kResidentWidthA) P.variant = kResidentA;
@@ -82,6 +83,7 @@ ResidentPlan plan_resident(const std::vector<ResidentInstance>& insts, const std
         }
     }
     if (resident_lds_bytes(P.lds_rows, P.max_halo, P.waves) > max_lds) return none;
+    P.by_start = resident_by_start(int(P.wgs.size()), P.max_cluster, cus);
     for (ResidentWg& W : P.wgs) W.pause_z = exchange_pause_z(W.cluster, P.waves < kGroupSlices, P.max_halo > 64 * (P.waves - 1));
     return P;
 }
