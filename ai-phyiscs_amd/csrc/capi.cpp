@@ -300,6 +300,13 @@ int chysx_cloth_set_resident_solve(chysx_cloth* sim, int mode) {
         sim->sim.problem().set_resident_solve(mode);
     });
 }
+int chysx_cloth_solve_form(const chysx_cloth* sim, int* out) {
+    return guard([&] {
+        need(sim, "simulator");
+        need(out, "out");
+        *out = const_cast<chysx_cloth*>(sim)->sim.problem().solve_form();
+    });
+}
 int chysx_cloth_set_pin_projection(chysx_cloth* sim, int on) {
     return guard([&] {
         need(sim, "sim");
@@ -545,6 +552,13 @@ int chysx_batch_set_resident_solve(chysx_batch* b, int mode) {
     return guard([&] {
         need(b, "batch");
         b->batch.problem().set_resident_solve(mode);
+    });
+}
+int chysx_batch_solve_form(const chysx_batch* b, int* out) {
+    return guard([&] {
+        need(b, "batch");
+        need(out, "out");
+        *out = const_cast<chysx_batch*>(b)->batch.problem().solve_form();
     });
 }
 int chysx_batch_set_pin_projection(chysx_batch* b, int on) {

@@ -616,6 +616,11 @@ void Problem::launch_resident(float dt, const DevExt& ext, hipStream_t s) {
     });
 }
 
+Problem::SolveForm Problem::next_form() const {
+    if (res_mode_ == 0) return kFormStreaming;
+    return res_.variant != kResidentNone ? kFormResident : sweep_.groups != 0 ? kFormSweep : kFormStreaming;
+}
+
 void Problem::check_resident(bool running) const {
     for (int k = 0; k < ninst_; ++k)
         if (host_states_[k].status != kConverged && host_states_[k].status != kStopped &&
@@ -1174,13 +1179,15 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
     proj_ran_ = false;
     start_r_ready_ = false;
     const bool ws_on = ws_mode_ != kWarmPrevious || ws_train_;
-    if (resident() || sweeps()) {
+    const SolveForm form = next_form();
+    if (form != kFormStreaming) {
         // the solve is launched directly, not as a graph, so a capture is refused here
         hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
         check_hip(hipStreamIsCapturing(s, &capturing), "hipStreamIsCapturing");
         if (capturing != hipStreamCaptureStatusNone)
             throw std::runtime_error("step: the stream is being captured; a step cannot be part of a graph");
     }
+    form_ = form;
     // Every instance at a fixed iteration count (tol == 0): the number of
     // rounds is known, so the whole solve is enqueued without a poll.
     bool fixed = !ws_on && !params_h_.empty();
@@ -1196,16 +1203,15 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
         // long fixed solves replay the chunk graphs instead, so a graph never
         // holds more than kStepGraphMaxChunks chunks
         const int chunks = std::max(1, (fixed_iters + 2 + kChunkIters - 1) / kChunkIters);
-        resident_step_ = resident() || sweeps();
-        if (resident()) {
+        if (form == kFormResident) {
             launch_assemble(dt, ext, s);
             launch_resident(dt, ext, s);
-        } else if (!sweeps() && chunks <= kStepGraphMaxChunks) {
+        } else if (form == kFormStreaming && chunks <= kStepGraphMaxChunks) {
             launch_fixed_step_graph(dt, ext, chunks, s);
         } else {
             launch_assemble(dt, ext, s);
             launch_pcg_start(s);
-            if (sweeps()) launch_sweep(s);
+            if (form == kFormSweep) launch_sweep(s);
             else launch_pcg_chunks(s, chunks);
             launch_pcg_residual(geom(), matrix(), vectors(), state_.data(), 1, s);
             launch_pcg_reduce(state_.data(), params_.data(), partials_.data(), ninst_, geom().ngroups, kPhaseFinal,
@@ -1223,7 +1229,7 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
     }
     launch_assemble(dt, ext, s);
     if (ws_on && hist_n_ >= 2) warm_start_stage(dt, ext, s);
-    if (resident()) {
+    if (form == kFormResident) {
         launch_resident(dt, ext, s);
         check_hip(hipStreamSynchronize(s), "hipStreamSynchronize(solve)");
         check_resident();
@@ -1240,10 +1246,10 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
     int chunks = std::max(1, (last_iters_ + 2 + kChunkIters - 1) / kChunkIters);
     int guard = 0;
     for (;;) {
-        if (sweeps()) launch_sweep(s);
+        if (form == kFormSweep) launch_sweep(s);
         else launch_pcg_chunks(s, chunks);
         read_states(s);
-        if (sweeps()) check_resident(true);
+        if (form == kFormSweep) check_resident(true);
         if (all_done()) break;
         chunks = 1;
         if (++guard > (1 << 22)) throw std::runtime_error("PCG did not terminate");
@@ -1316,7 +1322,7 @@ void Problem::resolve_stats() const {
     if (!stats_pending_) return;
     check_hip(hipEventSynchronize(done_event_), "hipEventSynchronize(step)");
     stats_pending_ = false;
-    if (resident_step_) check_resident();
+    if (form_ != kFormStreaming) check_resident();
     for (int k = 0; k < ninst_; ++k)
         if (host_states_[k].status == kRunning)
             throw std::runtime_error("PCG: a fixed-iteration solve did not end within its enqueued rounds");

@@ -309,10 +309,11 @@ public:
         res_mode_ = mode;
         destroy_graph();
     }
-    bool resident() const { return res_mode_ != 0 && res_.variant != kResidentNone; }
-    // A single cloth too large for that whose vectors fit the chip: its
-    // iterations run in one launch (pcg_sweep.hpp).
-    bool sweeps() const { return res_mode_ != 0 && sweep_.groups != 0; }
+    // How the latest step solved: with the kernels that stream the matrix, in
+    // one launch, or (a single cloth too large for that whose vectors fit the
+    // chip) with its iterations in one launch.
+    enum SolveForm : int { kFormStreaming = 0, kFormResident = 1, kFormSweep = 2 };
+    int solve_form() const { return form_; }
 
     const LaunchConfig& launch_config() const { return cfg_; }
     void set_launch_config(const LaunchConfig& c);
@@ -346,6 +347,8 @@ private:
     void launch_sweep(hipStream_t s);
     // Assembly and the resident solve, which ends with finalize; no host wait.
     void launch_resident(float dt, const DevExt& ext, hipStream_t s);
+    // The form of the next step's solve.
+    SolveForm next_form() const;
     // Throws when a solve lost a workgroup (or, unless `running`, has not ended).
     void check_resident(bool running = false) const;
     void train_after_solve(bool ws_on, hipStream_t s);
@@ -401,7 +404,7 @@ private:
 
     // resident solve
     mutable int res_mode_ = -1;
-    bool resident_step_ = false;  // the enqueued step's solve is a resident one
+    SolveForm form_ = kFormStreaming;  // of the latest step
     ResidentView res_{};
     DeviceArray<ResidentWg> res_wgs_;
     DeviceArray<uint16_t> res_loc_;

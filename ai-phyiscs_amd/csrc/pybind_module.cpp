@@ -27,6 +27,8 @@ void check(int rc) {
     throw std::runtime_error(msg);
 }
 
+const char* solve_form_name(int form) { return form == 1 ? "one_launch" : form == 2 ? "sweep" : "streaming"; }
+
 using IntArr = py::array_t<int32_t, py::array::c_style | py::array::forcecast>;
 using FltArr = py::array_t<float, py::array::c_style | py::array::forcecast>;
 using DblArr = py::array_t<double, py::array::c_style | py::array::forcecast>;
@@ -423,6 +425,14 @@ PYBIND11_MODULE(_chysx_native, m) {
             [](Sim& s, int mode) { check(chysx_cloth_set_resident_solve(s.p(), mode)); }, py::arg("mode"),
             "-1: the whole solve in one launch where the problem fits it; 0: never (speed only, the same bits).")
         .def(
+            "solve_form",
+            [](Sim& s) {
+                int form = 0;
+                check(chysx_cloth_solve_form(s.p(), &form));
+                return solve_form_name(form);
+            },
+            "How the latest step solved: 'streaming', 'one_launch' or 'sweep' (the iterations in one launch).")
+        .def(
             "set_pin_projection", [](Sim& s, bool on) { check(chysx_cloth_set_pin_projection(s.p(), on ? 1 : 0)); },
             py::arg("on"),
             "True: pins are constraints (each pinned particle ends every step exactly at its target); False "
@@ -671,6 +681,12 @@ PYBIND11_MODULE(_chysx_native, m) {
         .def(
             "set_resident_solve",
             [](Batch& b, int mode) { check(chysx_batch_set_resident_solve(b.h, mode)); }, py::arg("mode"))
+        .def("solve_form",
+             [](Batch& b) {
+                 int form = 0;
+                 check(chysx_batch_solve_form(b.h, &form));
+                 return solve_form_name(form);
+             })
         .def(
             "set_pin_projection",
             [](Batch& b, bool on) { check(chysx_batch_set_pin_projection(b.h, on ? 1 : 0)); }, py::arg("on"))

@@ -201,6 +201,9 @@ int chysx_cloth_set_pin_projection(chysx_cloth* sim, int on);
  * the kernels that stream the matrix; 2: as -1, with a start-up wait of no
  * length, after which one workgroup solves alone (tests).  Same bits. */
 int chysx_cloth_set_resident_solve(chysx_cloth* sim, int mode);
+/* How the latest step solved: 0 with the kernels that stream the matrix (also
+ * before the first step), 1 in one launch, 2 with the iterations in one launch. */
+int chysx_cloth_solve_form(const chysx_cloth* sim, int* out);
 int chysx_cloth_pin_projection(const chysx_cloth* sim, int* out);
 /* Per-element stiffness (one value per spring in edge order / per triangle). */
 int chysx_cloth_set_spring_stiffnesses(chysx_cloth* sim, const float* k, int n);
@@ -263,6 +266,8 @@ int chysx_batch_set_split_advance(chysx_batch* b, int mode);
 int chysx_batch_set_pin_projection(chysx_batch* b, int on);
 /* Where the solves run (as chysx_cloth_set_resident_solve). */
 int chysx_batch_set_resident_solve(chysx_batch* b, int mode);
+/* How the latest step solved (as chysx_cloth_solve_form). */
+int chysx_batch_solve_form(const chysx_batch* b, int* out);
 int chysx_batch_stats(const chysx_batch* b, int index, int* iters, int* restarts, int* status, double* relres);
 /* Number of cloths added to the batch. */
 int chysx_batch_num_cloths(const chysx_batch* b, int* n);

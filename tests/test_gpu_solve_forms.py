@@ -8,6 +8,9 @@ import pytest
 
 from chysx import scenes
 from chysx.harness import make_batch, make_sim
+from test_gpu_resident import CASES as ONE_LAUNCH
+from test_gpu_resident import fan
+from test_gpu_sweep import CASES as SWEEP
 
 pytestmark = pytest.mark.gpu
 
@@ -35,18 +38,24 @@ def mesh(w, h=None, crossed=False, seed=None):
                         pos[pins].copy(), 1.0e6, 1.0e3, 1.0e3, None, 1.0 / 60.0, 4)
 
 
-def assert_same_bits(make, steps=2, modes=(-1,)):
-    """Positions, velocities and statistics of `steps` steps under mode 0 and the others."""
+def handle(g):
+    return g.sim if hasattr(g, "sim") else g.batch
+
+
+def assert_same_bits(make, form, steps=2, modes=(-1,)):
+    """Positions, velocities and statistics of `steps` steps under mode 0 and the
+    others, which solve in form `form`."""
     out = {}
     for mode in (0, *modes):
         g = make()
-        h = g.sim if hasattr(g, "sim") else g.batch
+        h = handle(g)
         h.set_resident_solve(mode)
         rows = []
         for _ in range(steps):
             h.step(1.0 / 60.0)
             rows += [g.pos.cpu().numpy(), g.vel.cpu().numpy(),
                      [h.last_solve_stats()] if hasattr(g, "sim") else [h.stats(k) for k in range(h.num_cloths())]]
+            assert h.solve_form() == ("streaming" if mode == 0 else form)
         assert np.isfinite(rows[-3]).all()
         out[mode] = rows
     for mode in modes:
@@ -70,7 +79,7 @@ BATCHES = {
 @pytest.mark.parametrize("name", BATCHES)
 def test_batch_beyond_the_compute_units(cuda, name):
     sc = BATCHES[name]()
-    assert_same_bits(lambda: make_batch(sc, tol=0.0, max_iter=11))
+    assert_same_bits(lambda: make_batch(sc, tol=0.0, max_iter=11), "one_launch")
     b = make_batch(sc, tol=0.0, max_iter=11)
     b.batch.set_blocking_step(True)
     b.batch.step(1.0 / 60.0)
@@ -78,3 +87,63 @@ def test_batch_beyond_the_compute_units(cuda, name):
     b.batch.step(1.0 / 60.0)
     # milliseconds; half a second when workgroups wait for ones that cannot start
     assert time.perf_counter() - t < 0.3
+
+
+@pytest.mark.parametrize("cases, name", [(c, n) for c in (ONE_LAUNCH, SWEEP) for n in c],
+                         ids=lambda v: v if isinstance(v, str) else "")
+def test_the_form_that_solves(cuda, cases, name):
+    """The meshes that are compared with the streaming kernels do take the other forms."""
+    h = handle(cases[name]())
+    h.step(1.0 / 60.0)
+    # too wide (fan12_bending's hub couples to 24 rows), or one row too many
+    assert h.solve_form() == ("streaming" if name in ("fan30", "fan12_bending", "1025") else
+                              "one_launch" if cases is ONE_LAUNCH else "sweep")
+
+
+def drape(w):
+    return lambda: make_sim(scenes.drape(w, seed=5), tol=0.0, max_iter=9, springs_active=False)
+
+
+def cloth(*a, tol=0.0, **kw):
+    return lambda: make_sim(mesh(*a, **kw), tol=tol, max_iter=9 if tol == 0.0 else 10000)
+
+
+def training():
+    from chysx.warmstart import load_params
+    g = make_sim(mesh(48), tol=1e-6)
+    g.sim.ws_set_params(load_params()[0])
+    g.sim.set_warm_start_mode("learned")
+    g.sim.ws_set_training(True, 1e-4)
+    return g
+
+
+SHAPES = {
+    # 9-float half groups: z received before the sums (from 61 workgroups), more
+    # than 64 groups, more than one round of looks for three values (from 95
+    # groups), the most workgroups there are, one row too many
+    "drape200": (drape(200), "one_launch"), "drape270": (drape(270), "one_launch"),
+    "drape320": (drape(320), "one_launch"), "drape362": (drape(362), "one_launch"),
+    "drape363": (drape(363), "streaming"),
+    # packed half groups (rows of up to 8 neighbours)
+    "crossed23": (cloth(23, crossed=True), "one_launch"), "crossed150": (cloth(150, crossed=True, tol=1e-6), "one_launch"),
+    "crossed362": (cloth(362, crossed=True), "one_launch"), "crossed363": (cloth(363, crossed=True), "streaming"),
+    # the widest rows of each kind, and wider ones
+    "fan16": (lambda: make_sim(fan(16, 5), tol=1e-6), "one_launch"),
+    "fan17": (lambda: make_sim(fan(17, 5), tol=1e-6), "streaming"),
+    "fan7_bending": (lambda: make_sim(fan(7, 90, bend=0.01), tol=1e-6), "one_launch"),
+    "fan8_bending": (lambda: make_sim(fan(8, 9, bend=0.01), tol=1e-6), "streaming"),
+    # whole groups: the most workgroups, long and narrow, any numbering
+    "512": (cloth(512), "one_launch"), "16x4096": (cloth(16, 4096), "one_launch"),
+    "4096x16": (cloth(4096, 16), "one_launch"), "shuffled64": (cloth(64, seed=3, tol=1e-6), "one_launch"),
+    "shuffled128": (cloth(128, seed=3), "streaming"),
+    # the sweep beyond squares; boundary rows that no longer fit
+    "700x1400": (cloth(700, 1400), "sweep"), "300x2000": (cloth(300, 2000, tol=1e-4), "sweep"),
+    "1400x700": (cloth(1400, 700), "streaming"), "shuffled520": (cloth(520, seed=3), "streaming"),
+    "training": (training, "one_launch"),
+}
+
+
+@pytest.mark.parametrize("name", SHAPES)
+def test_same_bits_as_the_streaming_kernels(cuda, name):
+    make, form = SHAPES[name]
+    assert_same_bits(make, form, steps=3 if name == "training" else 2)
