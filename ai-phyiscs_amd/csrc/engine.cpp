@@ -497,6 +497,7 @@ void Problem::build(const std::vector<const Instance*>& insts) {
 
 void Problem::make_resident(const std::vector<int>& cols) {
     res_ = ResidentView{};
+    res_min_iters_ = 0;
     sweep_ = SweepView{};
     int dev = 0, cus = 0, lds = 0;
     check_hip(hipGetDevice(&dev), "hipGetDevice");
@@ -536,6 +537,7 @@ void Problem::make_resident(const std::vector<int>& cols) {
     res_.lds_bytes = resident_lds_bytes(P.lds_rows, P.max_halo, res_.block_waves);
     res_.max_cluster = P.max_cluster;
     res_.by_start = P.by_start ? 1 : 0;
+    res_min_iters_ = P.min_iters;
     res_.wgs = res_wgs_.data();
     res_.loc = res_loc_.data();
     res_.halo = res_halo_.data();
@@ -616,8 +618,8 @@ void Problem::launch_resident(float dt, const DevExt& ext, hipStream_t s) {
     });
 }
 
-Problem::SolveForm Problem::next_form() const {
-    if (res_mode_ == 0) return kFormStreaming;
+Problem::SolveForm Problem::next_form(int iters) const {
+    if (res_mode_ == 0 || (res_mode_ == -1 && iters < res_min_iters_)) return kFormStreaming;
     return res_.variant != kResidentNone ? kFormResident : sweep_.groups != 0 ? kFormSweep : kFormStreaming;
 }
 
@@ -1179,15 +1181,6 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
     proj_ran_ = false;
     start_r_ready_ = false;
     const bool ws_on = ws_mode_ != kWarmPrevious || ws_train_;
-    const SolveForm form = next_form();
-    if (form != kFormStreaming) {
-        // the solve is launched directly, not as a graph, so a capture is refused here
-        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-        check_hip(hipStreamIsCapturing(s, &capturing), "hipStreamIsCapturing");
-        if (capturing != hipStreamCaptureStatusNone)
-            throw std::runtime_error("step: the stream is being captured; a step cannot be part of a graph");
-    }
-    form_ = form;
     // Every instance at a fixed iteration count (tol == 0): the number of
     // rounds is known, so the whole solve is enqueued without a poll.
     bool fixed = !ws_on && !params_h_.empty();
@@ -1196,6 +1189,15 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
         fixed = fixed && q.tol2 == 0.0;
         fixed_iters = std::max(fixed_iters, q.max_iter);
     }
+    const SolveForm form = next_form(fixed || last_iters_ <= 0 ? fixed_iters : std::min(last_iters_, fixed_iters));
+    if (form != kFormStreaming) {
+        // the solve is launched directly, not as a graph, so a capture is refused here
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        check_hip(hipStreamIsCapturing(s, &capturing), "hipStreamIsCapturing");
+        if (capturing != hipStreamCaptureStatusNone)
+            throw std::runtime_error("step: the stream is being captured; a step cannot be part of a graph");
+    }
+    form_ = form;
     if (fixed && !blocking_) {
         // max_iter iterations plus a flush round and the advance that stops
         // the solve (rounds after the stop exit at once): the whole step,

@@ -347,8 +347,8 @@ private:
     void launch_sweep(hipStream_t s);
     // Assembly and the resident solve, which ends with finalize; no host wait.
     void launch_resident(float dt, const DevExt& ext, hipStream_t s);
-    // The form of the next step's solve.
-    SolveForm next_form() const;
+    // The form of the next step's solve, of about `iters` iterations.
+    SolveForm next_form(int iters) const;
     // Throws when a solve lost a workgroup (or, unless `running`, has not ended).
     void check_resident(bool running = false) const;
     void train_after_solve(bool ws_on, hipStream_t s);
@@ -405,6 +405,7 @@ private:
     // resident solve
     mutable int res_mode_ = -1;
     SolveForm form_ = kFormStreaming;  // of the latest step
+    int res_min_iters_ = 0;  // as ResidentPlan
     ResidentView res_{};
     DeviceArray<ResidentWg> res_wgs_;
     DeviceArray<uint16_t> res_loc_;

@@ -9,6 +9,7 @@
 #include <cmath>
 #include <cstdint>
 #include <functional>
+#include <limits>
 #include <vector>
 
 #include "cloth_kernels.hpp"
@@ -56,6 +57,7 @@ struct ResidentPlan {
     // Workgroups take their places in the order they start, not by their
     // number (resident_by_start).
     bool by_start = false;
+    int min_iters = 0;          // iterations from which the solve is faster in one launch (resident_min_iters)
     int lds_rows = 0;           // own and halo rows of the largest workgroup, and the zero row
     int max_halo = 0;
     std::vector<ResidentWg> wgs;
@@ -104,6 +106,35 @@ inline int exchange_pause(int wgs, bool halves) {
 inline int exchange_pause_z(int wgs, bool halves, bool wide) {
     const int p = exchange_pause(wgs, halves) - 6;
     return p <= 0 ? 0 : wide ? std::min(p, 6) : p;
+}
+
+// Iterations from which a batch is solved faster in one launch than by the
+// streaming kernels; kResidentNever: at no count.  clusters: the instances'
+// workgroups.  A batch whose workgroups all fit at once always is (1.2 to 3
+// times at 1 to 50 iterations), and so is one of single workgroups.  Beyond
+// that, whole groups lose at one iteration only (16 cloths of 256 x 256: 462
+// and 429 us; at 10 iterations 1.2 to 1.7 times as fast, at 50 1.4 to 2.4).
+// Half groups, on wide-row meshes, take twice the compute units for their
+// rows, and cloths that leave many of them unused gain nothing or lose (16
+// of 257 x 257, 130 workgroups each: 7.5 ms and 4.9 at 50 iterations).
+// Microseconds an iteration of the two forms, fitted at 2 to 256 workgroups a
+// cloth and 128 to 2048 groups (within 15%): 4.7 + 0.45 log2(workgroups) for
+// each generation of cloths that fit side by side, and 0.082 a group, at
+// least 20 to 24, or 33 from one group more than there are compute units on.
+// Loading the blocks costs the solve in one launch 0.35 us a group.
+constexpr int kResidentNever = std::numeric_limits<int>::max();
+inline int resident_min_iters(const std::vector<int>& clusters, int groups, bool halves, int cus) {
+    int wgs = 0, widest = 0;
+    double one = 0.0;
+    for (int c : clusters) {
+        wgs += c;
+        widest = std::max(widest, c);
+        one += (4.7 + 0.45 * std::log2(double(c))) / double(std::max(1, cus / c));
+    }
+    if (wgs <= cus || widest <= 1) return 0;
+    if (!halves) return 2;
+    const double streamed = std::max(groups <= cus ? 20.0 + 0.015 * groups : 33.0, 0.082 * groups);
+    return streamed <= one ? kResidentNever : int(std::ceil(0.35 * groups / (streamed - one)));
 }
 
 // One instance's rows for the plan.

@@ -84,6 +84,13 @@ ResidentPlan plan_resident(const std::vector<ResidentInstance>& insts, const std
     }
     if (resident_lds_bytes(P.lds_rows, P.max_halo, P.waves) > max_lds) return none;
     P.by_start = resident_by_start(int(P.wgs.size()), P.max_cluster, cus);
+    std::vector<int> clusters;
+    int groups = 0;
+    for (const ResidentInstance& I : insts) {
+        clusters.push_back((I.nslices + P.waves - 1) / P.waves);
+        groups += (I.nslices + kGroupSlices - 1) / kGroupSlices;
+    }
+    P.min_iters = resident_min_iters(clusters, groups, P.variant == kResidentB, cus);
     for (ResidentWg& W : P.wgs) W.pause_z = exchange_pause_z(W.cluster, P.waves < kGroupSlices, P.max_halo > 64 * (P.waves - 1));
     return P;
 }

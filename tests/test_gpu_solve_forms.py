@@ -147,3 +147,28 @@ SHAPES = {
 def test_same_bits_as_the_streaming_kernels(cuda, name):
     make, form = SHAPES[name]
     assert_same_bits(make, form, steps=3 if name == "training" else 2)
+
+
+def test_form_of_a_batch_by_its_iterations(cuda):
+    """Wide-row cloths that need more workgroups than there are compute units:
+    in one launch only from a number of iterations on, and not at all where they leave most compute units unused."""
+    def forms(sc, steps=1, **kw):
+        b = make_batch(sc, **kw)
+        out = []
+        for _ in range(steps):
+            b.batch.step(1.0 / 60.0)
+            out.append(b.batch.solve_form())
+        return out
+    many = [mesh(128, crossed=True) for _ in range(12)]
+    assert forms(many, tol=0.0, max_iter=2) == ["streaming"]
+    assert forms(many, tol=0.0, max_iter=50) == ["one_launch"]
+    assert forms(many, steps=2, tol=1e-6, max_iter=3) == ["streaming", "streaming"]
+    # with a tolerance, by the iterations of the step before: 6 for these cloths
+    b = make_batch(many, tol=1e-6)
+    before = 10000
+    for _ in range(5):
+        b.batch.step(1.0 / 60.0)
+        assert b.batch.solve_form() == ("one_launch" if before >= 6 else "streaming")
+        before = max(b.batch.stats(k)["iters"] for k in range(12))
+    assert forms([mesh(257, crossed=True) for _ in range(3)], tol=0.0, max_iter=50) == ["streaming"]
+    assert_same_bits(lambda: make_batch(many, tol=0.0, max_iter=50), "one_launch")

@@ -32,3 +32,15 @@ def test_every_batch_comes_to_run(compiled):
     assert rows["two198"][0] == 0 and rows["two198"][2] > 0
     assert rows["sixteen130"][2] > 0
     assert rows["uneven16"][0] == 1 and rows["one256"][0] == 1
+
+
+def test_batches_that_the_streaming_kernels_solve_faster(compiled):
+    """What fits at once always goes in one launch; beyond, it depends on the use of the compute units."""
+    rows = {r.split()[0]: [int(v) for v in r.split()[1:]] for r in compiled("min_iters").splitlines()}
+    never = 2 ** 31 - 1
+    for name in ("1x256", "5x44", "2000x1"):
+        assert rows[name] == [0, 0]
+    for name in ("3x130", "8x130", "16x130", "8x176"):  # measured 0.65 to 0.87 times as fast at 50 iterations
+        assert rows[name] == [never, 2]
+    for name in ("2x130", "16x64", "64x32", "128x20", "8x256", "4096x2"):  # 1.08 to 1.7 times as fast at 50
+        assert 1 < rows[name][0] <= 25 and rows[name][1] == 2
