@@ -175,6 +175,7 @@ Problem::~Problem() {
     destroy_graph();
     if (cap_stream_) (void)hipStreamDestroy(cap_stream_);
     if (host_states_) (void)hipHostFree(host_states_);
+    if (gate_device_ >= 0) leave_resident_gate(gate_device_, this);
     if (done_event_) (void)hipEventDestroy(done_event_);
 }
 
@@ -512,6 +513,7 @@ void Problem::make_resident(const std::vector<int>& cols) {
     const ResidentPlan P = plan_resident(insts, slice_ptr_h_, cols, block_floats(), cus, lds - kResidentStaticLds);
     if (P.variant == kResidentNone || P.wgs.empty()) {
         make_sweep(cols, std::min(cus, kResidentMaxWgs), lds);
+        if (sweep_.groups != 0) enter_gate(dev, gate_weight(sweep_.nwg, sweep_.nwg, true, cus), gate_room(cus));
         return;
     }
     hipStream_t s = nullptr;
@@ -538,6 +540,7 @@ void Problem::make_resident(const std::vector<int>& cols) {
     res_.max_cluster = P.max_cluster;
     res_.by_start = P.by_start ? 1 : 0;
     res_min_iters_ = P.min_iters;
+    enter_gate(dev, gate_weight(res_.nwg, P.max_cluster, P.by_start, cus), gate_room(cus));
     res_.wgs = res_wgs_.data();
     res_.loc = res_loc_.data();
     res_.halo = res_halo_.data();
@@ -550,6 +553,18 @@ void Problem::make_resident(const std::vector<int>& cols) {
     res_.ticket = res_ticket_.data();
     res_.meet_polls = kResidentMeetPolls;
     res_.variant = P.variant;
+}
+
+void Problem::enter_gate(int device, int weight, int room) {
+    if (gate_device_ >= 0 && gate_device_ != device) leave_resident_gate(gate_device_, this);
+    gate_device_ = device;
+    gate_weight_ = weight;
+    gate_room_ = room;
+    make_done_event();
+}
+
+void Problem::make_done_event() {
+    if (!done_event_) check_hip(hipEventCreateWithFlags(&done_event_, hipEventDisableTiming), "hipEventCreate");
 }
 
 void Problem::make_sweep(const std::vector<int>& cols, int max_wgs, int lds) {
@@ -598,7 +613,7 @@ void Problem::launch_sweep(hipStream_t s) {
     SweepView R = sweep_;
     if (res_mode_ == 2) R.meet_polls = 0;
     const LaunchGeom g = geom();
-    with_resident_gate(R.nwg, s, [&] { launch_pcg_sweep(R, g, matrix(), vectors(), state_.data(), params_.data(), s); });
+    with_resident_gate(gated(), s, [&] { launch_pcg_sweep(R, g, matrix(), vectors(), state_.data(), params_.data(), s); });
     bool checks = false;
     for (const InstParams& q : params_h_) checks = checks || q.tol2 > 0.0;
     if (!checks) return;
@@ -612,7 +627,7 @@ void Problem::launch_resident(float dt, const DevExt& ext, hipStream_t s) {
     if (res_mode_ == 2) R.meet_polls = 0;
     const int given_r = start_r_ready_ ? 1 : 0;
     start_r_ready_ = false;
-    with_resident_gate(R.max_cluster, s, [&] {
+    with_resident_gate(gated(), s, [&] {
         launch_pcg_resident(R, geom(), matrix(), vectors(), ext, mesh(), state_.data(), host_states_, params_.data(),
                             dt, given_r, s);
     });
@@ -1223,8 +1238,11 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
                 hipMemcpyAsync(host_states_, state_.data(), sizeof(InstState) * ninst_, hipMemcpyDeviceToHost, s),
                 "hipMemcpyAsync(states)");
         }
-        if (!done_event_) check_hip(hipEventCreateWithFlags(&done_event_, hipEventDisableTiming), "hipEventCreate");
-        check_hip(hipEventRecord(done_event_, s), "hipEventRecord(step)");
+        // a gated solve that ends the step has recorded the event
+        if (form != kFormResident || gate_weight_ == 0) {
+            make_done_event();
+            check_hip(hipEventRecord(done_event_, s), "hipEventRecord(step)");
+        }
         stats_pending_ = true;
         last_iters_ = fixed_iters;
         return;

@@ -342,6 +342,9 @@ private:
     // columns on the host.
     void make_resident(const std::vector<int>& cols);
     void make_sweep(const std::vector<int>& cols, int max_wgs, int lds);
+    void enter_gate(int device, int weight, int room);
+    void make_done_event();
+    GatedLaunch gated() const { return GatedLaunch{this, done_event_, gate_device_, gate_weight_, gate_room_}; }
     // The iterations of a started solve until its next true-residual check,
     // and that check; no host wait.
     void launch_sweep(hipStream_t s);
@@ -424,7 +427,8 @@ private:
     int last_iters_ = 0;
     bool blocking_ = false;
     mutable bool stats_pending_ = false;  // host_states_ is being copied for an enqueued step
-    hipEvent_t done_event_ = nullptr;     // recorded after that copy
+    hipEvent_t done_event_ = nullptr;     // recorded after that copy, and behind every gated launch
+    int gate_device_ = -1, gate_weight_ = 0, gate_room_ = 0;  // resident_gate.hpp
 
     LaunchConfig cfg_;
     std::vector<TuneSample> tune_log_;

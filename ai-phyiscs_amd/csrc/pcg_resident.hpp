@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "cloth_kernels.hpp"
+#include "resident_gate.hpp"
 
 namespace chysx_amd {
 
@@ -78,7 +79,6 @@ struct ResidentPlan {
 // 0.8 ms by number).
 // By number (false): an instance lies evenly over the XCDs, and the first one
 // that has not met is next in line on each of them, so it always comes to run.
-constexpr int kXcds = 8;
 inline bool resident_by_start(int wgs, int max_cluster, int cus) {
     return max_cluster > 1 && (wgs <= cus || max_cluster <= cus / kXcds);
 }
@@ -199,8 +199,16 @@ void launch_pcg_resident(const ResidentView& R, const LaunchGeom& g, const DevMa
                          const DevExt& e, const DevMesh& m, InstState* st, InstState* host_st,
                          const InstParams* params, float dt, int start_given_r, hipStream_t s);
 
-// Runs `enqueue`, which puts a resident solve on stream s, in turn with the
-// device's other ones when its instances span many workgroups.
-void with_resident_gate(int max_cluster, hipStream_t s, const std::function<void()>& enqueue);
+// Runs `enqueue`, which puts a launch of `owner` on stream s, behind those of
+// the device's launches in flight that it cannot run beside, and records
+// `done` after it.  weight and room: gate_weight, gate_room.
+struct GatedLaunch {
+    const void* owner;
+    hipEvent_t done;
+    int device, weight, room;
+};
+void with_resident_gate(const GatedLaunch& L, hipStream_t s, const std::function<void()>& enqueue);
+// The owner's launches have run, and its event goes away.
+void leave_resident_gate(int device, const void* owner);
 
 }  // namespace chysx_amd

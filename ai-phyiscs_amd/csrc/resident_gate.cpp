@@ -1,4 +1,6 @@
 // SPDX-License-Identifier: Apache-2.0
+#include "resident_gate.hpp"
+
 #include <hip/hip_runtime.h>
 
 #include <functional>
@@ -13,44 +15,45 @@ namespace chysx_amd {
 
 namespace {
 
-// Launches whose instances span more than kFreeCluster workgroups run one
-// after the other on a device, whatever their streams: two that each hold part
-// of the compute units while they wait for the rest would not meet.  Smaller
-// ones never hold enough of them (at most 32 hardware queues with 7 waiting
-// workgroups each, of 256 compute units) and stay free.
-constexpr int kFreeCluster = 8;
 constexpr int kMaxDevices = 64;
 struct Gate {
     std::mutex lock;
-    hipEvent_t last = nullptr;  // the latest gated launch
-    hipStream_t stream = nullptr;
+    GateBook<hipEvent_t> book;
 };
-Gate& gate_of_device() {
+Gate& gate_of(int device) {
     static Gate gates[kMaxDevices];
-    int dev = 0;
-    const hipError_t err = hipGetDevice(&dev);
-    if (err != hipSuccess) throw_hip(err, "hipGetDevice");
-    if (dev < 0 || dev >= kMaxDevices) throw std::runtime_error("chysx: device index out of range");
-    return gates[dev];
+    if (device < 0 || device >= kMaxDevices) throw std::runtime_error("chysx: device index out of range");
+    return gates[device];
 }
 
 }  // namespace
 
-void with_resident_gate(int max_cluster, hipStream_t s, const std::function<void()>& enqueue) {
-    if (max_cluster <= kFreeCluster) {
+void with_resident_gate(const GatedLaunch& L, hipStream_t s, const std::function<void()>& enqueue) {
+    if (L.weight <= 0) {
         enqueue();
         return;
     }
     auto check = [](hipError_t err, const char* what) {
         if (err != hipSuccess) throw_hip(err, what);
     };
-    Gate& G = gate_of_device();
+    Gate& G = gate_of(L.device);
     const std::lock_guard<std::mutex> hold(G.lock);
-    if (!G.last) check(hipEventCreateWithFlags(&G.last, hipEventDisableTiming), "hipEventCreate(resident solve)");
-    else if (G.stream != s) check(hipStreamWaitEvent(s, G.last, 0), "hipStreamWaitEvent(resident solve)");
+    const auto waits = G.book.admit(L.owner, L.done, L.weight, L.room, [&](hipEvent_t e) {
+        const hipError_t err = hipEventQuery(e);
+        if (err == hipSuccess) return true;
+        if (err != hipErrorNotReady) throw_hip(err, "hipEventQuery(solve in flight)");
+        (void)hipGetLastError();  // not an error of a later launch
+        return false;
+    });
+    for (hipEvent_t e : waits) check(hipStreamWaitEvent(s, e, 0), "hipStreamWaitEvent(solve in flight)");
     enqueue();
-    check(hipEventRecord(G.last, s), "hipEventRecord(resident solve)");
-    G.stream = s;
+    check(hipEventRecord(L.done, s), "hipEventRecord(solve)");
+}
+
+void leave_resident_gate(int device, const void* owner) {
+    Gate& G = gate_of(device);
+    const std::lock_guard<std::mutex> hold(G.lock);
+    G.book.forget(owner);
 }
 
 }  // namespace chysx_amd

@@ -172,3 +172,32 @@ def test_form_of_a_batch_by_its_iterations(cuda):
         before = max(b.batch.stats(k)["iters"] for k in range(12))
     assert forms([mesh(257, crossed=True) for _ in range(3)], tol=0.0, max_iter=50) == ["streaming"]
     assert_same_bits(lambda: make_batch(many, tol=0.0, max_iter=50), "one_launch")
+
+
+def test_wide_and_small_solves_on_several_streams(cuda):
+    """A cloth that takes every compute unit beside batches whose cloths span a
+    few workgroups, each on a stream of its own: the results of each alone, and
+    no start-up wait that runs out (half a second each)."""
+    import torch
+    small = [mesh(w) for w in [40, 64, 90] * 30]
+    makes = [lambda: make_sim(mesh(512), tol=0.0, max_iter=20), lambda: make_batch(small, tol=0.0, max_iter=15),
+             lambda: make_sim(mesh(513), tol=0.0, max_iter=10), lambda: make_batch(small[:40], tol=0.0, max_iter=40)]
+    alone = []
+    for make in makes:
+        g = make()
+        for _ in range(9):
+            handle(g).step(1.0 / 60.0)
+        alone.append(g.pos.cpu().numpy())
+    gs = [make() for make in makes]
+    streams = [torch.cuda.Stream() for _ in gs]
+    for g in gs:
+        handle(g).step(1.0 / 60.0)
+    torch.cuda.synchronize()
+    t = time.perf_counter()
+    for _ in range(8):
+        for g, s in zip(gs, streams):
+            handle(g).step(1.0 / 60.0, s.cuda_stream)
+    torch.cuda.synchronize()
+    assert time.perf_counter() - t < 0.4
+    for g, want in zip(gs, alone):
+        np.testing.assert_array_equal(g.pos.cpu().numpy(), want)

@@ -44,3 +44,8 @@ def test_batches_that_the_streaming_kernels_solve_faster(compiled):
         assert rows[name] == [never, 2]
     for name in ("2x130", "16x64", "64x32", "128x20", "8x256", "4096x2"):  # 1.08 to 1.7 times as fast at 50
         assert 1 < rows[name][0] <= 25 and rows[name][1] == 2
+
+
+def test_solves_in_flight_together_leave_room(compiled):
+    """Launches that may be under way together never hold a whole XCD with waiting workgroups."""
+    assert compiled("gate").startswith("ok ")
