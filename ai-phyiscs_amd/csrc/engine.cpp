@@ -815,7 +815,10 @@ void Problem::set_launch_config(const LaunchConfig& c) {
         // A new storage reuses the value and diagonal buffers with another
         // layout.  Padding entries must read as zero blocks (the branch-free
         // SpMV multiplies them), and assembly writes only real entries, so
-        // clear what the old layout left behind.
+        // clear what the old layout left behind.  An enqueued step still reads
+        // both, and the plan, exchange words and arrival counts replaced
+        // below, on a stream that the null stream may not be ordered with.
+        if (stats_pending_) check_hip(hipEventSynchronize(done_event_), "hipEventSynchronize(enqueued step)");
         val_.zero(nullptr);
         diag_.zero(nullptr);
         check_hip(hipStreamSynchronize(nullptr), "hipStreamSynchronize(storage change)");

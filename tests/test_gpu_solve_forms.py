@@ -201,3 +201,25 @@ def test_wide_and_small_solves_on_several_streams(cuda):
     assert time.perf_counter() - t < 0.4
     for g, want in zip(gs, alone):
         np.testing.assert_array_equal(g.pos.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("w", [60, 530])
+def test_storage_changed_behind_an_enqueued_step(cuda, w):
+    """A change of the matrix storage waits for the step that was enqueued
+    before it, on a stream of its own."""
+    import torch
+    def run(wait):
+        g = make_sim(mesh(w), tol=0.0, max_iter=400)
+        s = torch.cuda.Stream()
+        torch.cuda.synchronize()
+        for storage in (dict(spmv_symmetric=0), dict(spmv_symmetric=1, spmv_packed=1), dict(spmv_symmetric=1, spmv_packed=0)):
+            g.sim.step(1.0 / 60.0, s.cuda_stream)
+            if wait:
+                torch.cuda.synchronize()
+            g.sim.set_launch_config(storage)
+        g.sim.step(1.0 / 60.0, s.cuda_stream)
+        torch.cuda.synchronize()
+        return g.pos.cpu().numpy(), g.sim.last_solve_stats()
+    (a, sa), (b, sb) = run(False), run(True)
+    np.testing.assert_array_equal(a, b)
+    assert sa == sb and np.isfinite(a).all()
