@@ -194,6 +194,7 @@ void Problem::build(const std::vector<const Instance*>& insts) {
         check_hip(hipEventSynchronize(done_event_), "hipEventSynchronize(previous step)");
         stats_pending_ = false;
     }
+    raise_if_lost();
     destroy_graph();
     built_ = false;
     ninst_ = int(insts.size());
@@ -486,8 +487,12 @@ void Problem::build(const std::vector<const Instance*>& insts) {
     shapes_h_.clear();
     if (host_states_) (void)hipHostFree(host_states_);
     host_states_ = nullptr;
-    check_hip(hipHostMalloc(reinterpret_cast<void**>(&host_states_), sizeof(InstState) * std::max(ninst_, 1)),
+    notice_ = nullptr;
+    const size_t state_bytes = sizeof(InstState) * size_t(std::max(ninst_, 1));
+    check_hip(hipHostMalloc(reinterpret_cast<void**>(&host_states_), state_bytes + sizeof(ResidentNotice)),
               "hipHostMalloc(states)");
+    notice_ = reinterpret_cast<ResidentNotice*>(reinterpret_cast<char*>(host_states_) + state_bytes);
+    *notice_ = ResidentNotice{};
     std::memcpy(host_states_, st.data(), sizeof(InstState) * st.size());
     make_resident(sell_col);
     check_hip(hipStreamSynchronize(s), "hipStreamSynchronize(build)");
@@ -499,6 +504,7 @@ void Problem::build(const std::vector<const Instance*>& insts) {
 void Problem::make_resident(const std::vector<int>& cols) {
     res_ = ResidentView{};
     res_min_iters_ = 0;
+    res_lost_ = false;
     sweep_ = SweepView{};
     int dev = 0, cus = 0, lds = 0;
     check_hip(hipGetDevice(&dev), "hipGetDevice");
@@ -526,11 +532,7 @@ void Problem::make_resident(const std::vector<int>& cols) {
     res_zx_.resize(P.max_cluster > 1 ? size_t(n_pad_) * 2 : 1);
     res_slots_.resize(P.max_cluster > 1 ? resident_slot_words(nslices() / kGroupSlices) : 1);
     res_solo_.resize(P.max_cluster > 1 ? size_t(nslices()) * 3 : 1);
-    res_sync_.zero(s);
-    res_ticket_.zero(s);
-    res_zx_.zero(s);
-    res_slots_.zero(s);
-    check_hip(hipStreamSynchronize(s), "hipStreamSynchronize(resident plan)");
+    if (P.max_cluster > 1) clear_exchange(0);  // single workgroups exchange nothing
     res_.waves = P.waves;
     res_.block_waves = P.max_cluster > 1 ? P.waves : P.max_nslices;
     res_.nwg = int(P.wgs.size());
@@ -538,7 +540,6 @@ void Problem::make_resident(const std::vector<int>& cols) {
     res_.lds_x = resident_lds_x(P.lds_rows, P.max_halo);
     res_.lds_bytes = resident_lds_bytes(P.lds_rows, P.max_halo, res_.block_waves);
     res_.max_cluster = P.max_cluster;
-    res_.by_start = P.by_start ? 1 : 0;
     res_min_iters_ = P.min_iters;
     enter_gate(dev, gate_weight(res_.nwg, P.max_cluster, P.by_start, cus), gate_room(cus));
     res_.wgs = res_wgs_.data();
@@ -550,7 +551,7 @@ void Problem::make_resident(const std::vector<int>& cols) {
     res_.slots = res_slots_.data();
     res_.solo = res_solo_.data();
     res_.sync = res_sync_.data();
-    res_.ticket = res_ticket_.data();
+    res_.ticket = P.by_start ? res_ticket_.data() : nullptr;
     res_.meet_polls = kResidentMeetPolls;
     res_.variant = P.variant;
 }
@@ -586,10 +587,8 @@ void Problem::make_sweep(const std::vector<int>& cols, int max_wgs, int lds) {
     res_slots_.resize(sweep_slot_words(ngroups));
     res_solo_.resize(size_t(nslices()) * 3);
     res_sync_.resize(1);
-    res_zx_.zero(s);
-    res_slots_.zero(s);
-    res_sync_.zero(s);
     check_hip(hipStreamSynchronize(s), "hipStreamSynchronize(sweep plan)");
+    clear_exchange(0);
     sweep_.nwg = int(P.wgs.size());
     sweep_.ngroups = ngroups;
     sweep_.lds_rows = P.lds_rows;
@@ -634,17 +633,44 @@ void Problem::launch_resident(float dt, const DevExt& ext, hipStream_t s) {
 }
 
 Problem::SolveForm Problem::next_form(int iters) const {
-    if (res_mode_ == 0 || (res_mode_ == -1 && iters < res_min_iters_)) return kFormStreaming;
+    if (res_mode_ == 0 || res_lost_ || (res_mode_ == -1 && iters < res_min_iters_)) return kFormStreaming;
     return res_.variant != kResidentNone ? kFormResident : sweep_.groups != 0 ? kFormSweep : kFormStreaming;
 }
 
-void Problem::check_resident(bool running) const {
-    for (int k = 0; k < ninst_; ++k)
-        if (host_states_[k].status != kConverged && host_states_[k].status != kStopped &&
-            !(running && host_states_[k].status == kRunning)) {
-            res_mode_ = 0;  // the exchange words are in no known state
-            throw std::runtime_error("PCG: a solve lost one of its workgroups");
-        }
+void Problem::set_resident_solve(int mode) {
+    if (mode != -1 && mode != 0 && mode != 2 && mode != 4)
+        throw std::invalid_argument("resident solve: -1, 0, 2 or 4");
+    if (mode != 0 && (res_lost_ || mode == 4)) clear_exchange(mode == 4 ? 1u : 0u);
+    res_mode_ = mode;
+    destroy_graph();
+}
+
+void Problem::clear_exchange(unsigned lost) {
+    res_lost_ = false;
+    if (res_sync_.size() == 0) return;
+    if (stats_pending_) check_hip(hipEventSynchronize(done_event_), "hipEventSynchronize(enqueued step)");
+    hipStream_t s = nullptr;
+    std::vector<ResidentSync> sync(res_sync_.size(), ResidentSync{});
+    for (ResidentSync& q : sync) {
+        q.lost = lost;
+        q.notice = notice_;
+    }
+    res_sync_.assign(sync.data(), sync.size(), s);
+    if (res_ticket_.size() > 0) res_ticket_.zero(s);
+    res_zx_.zero(s);
+    res_slots_.zero(s);
+    check_hip(hipStreamSynchronize(s), "hipStreamSynchronize(exchange words)");
+}
+
+void Problem::raise_if_lost() const {
+    if (!notice_ || static_cast<volatile ResidentNotice*>(notice_)->lost == 0) return;
+    // steps enqueued behind the lost one give the same notice
+    if (stats_pending_) check_hip(hipEventSynchronize(done_event_), "hipEventSynchronize(enqueued step)");
+    stats_pending_ = false;
+    notice_->lost = 0;
+    res_lost_ = true;
+    throw std::runtime_error(
+        "PCG: a solve lost one of its workgroups; positions and velocities since that step are not valid");
 }
 
 void Problem::upload_params(const std::vector<const Instance*>& insts, hipStream_t s) {
@@ -1193,6 +1219,7 @@ void Problem::warm_start_stage(float dt, const DevExt& ext, hipStream_t s) {
 
 void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
     if (!built_ || ninst_ == 0) return;
+    raise_if_lost();
     wait_pending(s);
     stats_pending_ = false;
     ws_ran_ = false;
@@ -1255,7 +1282,7 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
     if (form == kFormResident) {
         launch_resident(dt, ext, s);
         check_hip(hipStreamSynchronize(s), "hipStreamSynchronize(solve)");
-        check_resident();
+        raise_if_lost();
         last_iters_ = 0;
         for (int k = 0; k < ninst_; ++k) last_iters_ = std::max(last_iters_, host_states_[k].iters);
         train_after_solve(ws_on, s);
@@ -1272,7 +1299,7 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
         if (form == kFormSweep) launch_sweep(s);
         else launch_pcg_chunks(s, chunks);
         read_states(s);
-        if (form == kFormSweep) check_resident(true);
+        raise_if_lost();
         if (all_done()) break;
         chunks = 1;
         if (++guard > (1 << 22)) throw std::runtime_error("PCG did not terminate");
@@ -1345,7 +1372,7 @@ void Problem::resolve_stats() const {
     if (!stats_pending_) return;
     check_hip(hipEventSynchronize(done_event_), "hipEventSynchronize(step)");
     stats_pending_ = false;
-    if (form_ != kFormStreaming) check_resident();
+    raise_if_lost();
     for (int k = 0; k < ninst_; ++k)
         if (host_states_[k].status == kRunning)
             throw std::runtime_error("PCG: a fixed-iteration solve did not end within its enqueued rounds");

@@ -304,11 +304,10 @@ public:
     // -1 where it fits, 0 never, 2 where it fits but with a start-up wait of
     // no length, so that an instance's first workgroup solves it alone (for
     // tests).  Results are the same bits.
-    void set_resident_solve(int mode) {
-        if (mode != -1 && mode != 0 && mode != 2) throw std::invalid_argument("resident solve: -1, 0 or 2");
-        res_mode_ = mode;
-        destroy_graph();
-    }
+    // 4: where it fits, with the exchange between workgroups marked as one
+    // that has lost a workgroup leaves it (for tests).  After a step has failed
+    // for that reason the streaming kernels take over until this is called.
+    void set_resident_solve(int mode);
     // How the latest step solved: with the kernels that stream the matrix, in
     // one launch, or (a single cloth too large for that whose vectors fit the
     // chip) with its iterations in one launch.
@@ -352,8 +351,11 @@ private:
     void launch_resident(float dt, const DevExt& ext, hipStream_t s);
     // The form of the next step's solve, of about `iters` iterations.
     SolveForm next_form(int iters) const;
-    // Throws when a solve lost a workgroup (or, unless `running`, has not ended).
-    void check_resident(bool running = false) const;
+    // Throws when a solve since the last call lost a workgroup, or was not
+    // started after one that did.
+    void raise_if_lost() const;
+    // The exchange words as before the first solve, with every instance marked `lost`.
+    void clear_exchange(unsigned lost);
     void train_after_solve(bool ws_on, hipStream_t s);
     // Fills the statistics of a step whose solver states the host has.
     void end_step(hipStream_t s);
@@ -406,7 +408,9 @@ private:
     DeviceArray<int> gactive_;  // batches: 1 per group of a running instance
 
     // resident solve
-    mutable int res_mode_ = -1;
+    int res_mode_ = -1;
+    mutable bool res_lost_ = false;  // a solve lost a workgroup: the exchange words are in no known state
+    ResidentNotice* notice_ = nullptr;  // behind host_states_
     SolveForm form_ = kFormStreaming;  // of the latest step
     int res_min_iters_ = 0;  // as ResidentPlan
     ResidentView res_{};

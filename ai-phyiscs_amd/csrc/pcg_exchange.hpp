@@ -99,12 +99,24 @@ __device__ __forceinline__ double slot_wait(const Cluster& C, const u64* w, unsi
     return __hiloint2double(int(unsigned(b)), int(unsigned(a)));
 }
 
+// A wait of the exchange ran out, in this launch or an earlier one.
+__device__ __forceinline__ void lost_exchange(ResidentSync* S) {
+    S->lost = 1;
+    __hip_atomic_store(&S->notice->lost, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // The instance's workgroups agree that they run: all of them have started, so
 // every wait that follows ends.  If they have not met within R.meet_polls (the
 // device's compute units are held by waiting workgroups of another process),
-// one of them solves the instance alone and the others leave.
+// one of them solves the instance alone and the others leave.  After a launch
+// that lost a workgroup all leave (a loss in this launch comes after all have
+// met, so they agree on that, too).
 enum Meeting : int { kMeetRun = 0, kMeetLeave = 1, kMeetAlone = 2 };
 __device__ int meet(ResidentSync* S, int cluster, int polls) {
+    if (S->lost != 0) {
+        lost_exchange(S);
+        return kMeetLeave;
+    }
     const u64 a = __hip_atomic_fetch_add(&S->arrived, u64(1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const u64 run = 2 * (a / u64(cluster) + 1);
     if ((a + 1) % u64(cluster) == 0) {

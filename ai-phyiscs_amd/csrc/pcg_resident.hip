@@ -302,7 +302,7 @@ __global__ __launch_bounds__(64 * NW) void pcg_resident_kernel(ResidentView R, L
     const int tid = threadIdx.x, wave = uniform_int(tid >> 6), lane = tid & 63;
     const int threads = int(blockDim.x);
     int wgi = blockIdx.x;
-    if (R.by_start) {  // places in the order of starting (plan_resident says when)
+    if (R.ticket != nullptr) {  // places in the order of starting (plan_resident says when)
         if (tid == 0)
             shared_int[0] = int(__hip_atomic_fetch_add(R.ticket, u64(1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) %
                                 u64(R.nwg));
@@ -582,8 +582,9 @@ __global__ __launch_bounds__(64 * NW) void pcg_resident_kernel(ResidentView R, L
     }
     if (!met_all) {
         if (tid == 0) {
-            mem.status = kResidentTimedOut;
-            host_st[W.inst].status = kResidentTimedOut;
+            mem.status = kResidentLost;
+            host_st[W.inst].status = kResidentLost;
+            lost_exchange(R.sync + W.inst);
         }
         return;
     }

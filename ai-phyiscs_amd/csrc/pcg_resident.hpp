@@ -150,18 +150,26 @@ struct ResidentInstance {
 ResidentPlan plan_resident(const std::vector<ResidentInstance>& insts, const std::vector<int>& slice_ptr,
                            const std::vector<int>& cols, int bs, int cus, int max_lds);
 
+// What the host has to know of solves that it may not ask for their outcome,
+// in pinned memory; stays until the host takes it back.
+struct ResidentNotice {
+    int lost;  // 1: a solve lost a workgroup, or was not started after one that did
+};
+
 // Start-up agreement of an instance's workgroups, kept in device memory across
-// launches (all zero at first).
+// launches (counts all zero at first).
 struct ResidentSync {
     unsigned long long arrived;   // workgroups started, over all launches
     unsigned long long decision;  // 2 L: launch L (1, 2, ...) runs; 2 L + 1: its workgroups did not meet in time
     unsigned epoch;               // last tag used in the exchange words
-    unsigned pad;
+    // 1: a wait of an exchange ran out.  Words with tags beyond the epoch may
+    // be there or still come, so no solve starts until the host has cleared them.
+    unsigned lost;
+    ResidentNotice* notice;
 };
 
 struct ResidentView {
     int variant, waves, block_waves, nwg, lds_rows, lds_x, lds_bytes, max_cluster;
-    int by_start;               // as ResidentPlan
     const ResidentWg* wgs;
     const uint16_t* loc;
     const int* halo;
@@ -171,7 +179,7 @@ struct ResidentView {
     unsigned long long* slots;  // partial sums: kinds x pieces x copies x 2 halves x groups words
     double* solo;               // 3 per slice: partial sums of an instance solved by one workgroup
     ResidentSync* sync;         // per instance
-    unsigned long long* ticket; // workgroups started, over all launches (by_start)
+    unsigned long long* ticket; // workgroups started, over all launches; null: places by number
     int meet_polls;             // bound of the start-up wait, in polls of about a microsecond
 };
 constexpr int kResidentKinds = 6;   // 0: p . Ap; 1, 2: r . z, |r|^2; 3 .. 5: start, check and report sums
@@ -188,9 +196,9 @@ inline size_t resident_slot_words(int ngroups) {
     return size_t(kResidentKinds) * kResidentPieces * kResidentCopies * 2 * size_t(ngroups);
 }
 
-// Status a solve is left with when a wait of the exchange ran out (reported
-// as an error by the host; it takes a lost workgroup).
-constexpr int kResidentTimedOut = 4;
+// Status of an instance whose solve lost a workgroup (a wait of the exchange
+// ran out); the host reports an error.
+constexpr int kResidentLost = 4;
 
 // Start residual, iterations, true-residual checks, report residual and
 // finalize of every instance, from the assembled system.  host_st: the solver

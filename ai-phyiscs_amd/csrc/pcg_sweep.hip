@@ -230,7 +230,7 @@ __global__ __launch_bounds__(kThreads) void pcg_sweep_kernel(SweepView R, Launch
         mem.rho = S.rho;
         mem.rr = S.rr;
         mem.beta = S.beta;
-        mem.status = ok ? S.status : kResidentTimedOut;
+        mem.status = S.status;
         mem.mode = S.mode;
         mem.iters = S.iters;
         mem.parity = S.parity;
@@ -238,6 +238,7 @@ __global__ __launch_bounds__(kThreads) void pcg_sweep_kernel(SweepView R, Launch
         mem.pend = S.pend;
         mem.defer = S.defer;
         mem.owed = S.status == kRunning ? 1 : 0;  // the check pass that follows owes its advance
+        if (!ok) lost_exchange(R.sync);
     };
     if (met == kMeetAlone) {
         S.slice0 = mem.slice0;

@@ -199,7 +199,11 @@ int chysx_cloth_set_pin_projection(chysx_cloth* sim, int on);
  * matrix in registers, for cloths it fits (up to 256 workgroups), or, for one
  * regularly triangulated cloth up to 1024x1024, its vectors; 0: always in
  * the kernels that stream the matrix; 2: as -1, with a start-up wait of no
- * length, after which one workgroup solves alone (tests).  Same bits. */
+ * length, after which one workgroup solves alone (tests).  Same bits.
+ * A solve whose workgroups lose each other ends after some seconds, and the
+ * step, the statistics or the next step report it as an error; later steps
+ * stream the matrix until this is called again.  4: as -1, marked as such a
+ * solve leaves it (tests). */
 int chysx_cloth_set_resident_solve(chysx_cloth* sim, int mode);
 /* How the latest step solved: 0 with the kernels that stream the matrix (also
  * before the first step), 1 in one launch, 2 with the iterations in one launch. */

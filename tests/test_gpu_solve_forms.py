@@ -223,3 +223,50 @@ def test_storage_changed_behind_an_enqueued_step(cuda, w):
     (a, sa), (b, sb) = run(False), run(True)
     np.testing.assert_array_equal(a, b)
     assert sa == sb and np.isfinite(a).all()
+
+
+LOST = {"one_launch": lambda: make_sim(mesh(60), tol=0.0, max_iter=20),
+        "one_launch_tol": lambda: make_sim(mesh(60), tol=1e-6),
+        "batch": lambda: make_batch([mesh(w) for w in (20, 60, 40)], tol=0.0, max_iter=20),
+        "sweep": lambda: make_sim(mesh(520), tol=0.0, max_iter=5),
+        "sweep_tol": lambda: make_sim(mesh(520), tol=1e-4)}
+
+
+@pytest.mark.parametrize("name", LOST)
+def test_lost_workgroup_is_reported_and_not_trusted(cuda, name):
+    """After a solve that lost a workgroup (mode 4 marks the exchange as such a
+    solve leaves it) no further one runs on its words: the error comes from the
+    step itself, from the statistics, or from the next step of a caller who asks
+    for none; then the streaming kernels take over, until the one-launch form is
+    asked for again."""
+    import torch
+    stats = (lambda h: h.last_solve_stats()) if name != "batch" else (lambda h: h.stats(0))
+    for ask in ("stats", "next step"):
+        g = LOST[name]()
+        h = handle(g)
+        form = name.split("_tol")[0].replace("batch", "one_launch")
+        h.step(1.0 / 60.0)
+        torch.cuda.synchronize()
+        assert h.solve_form() == form
+        h.set_resident_solve(4)
+        with pytest.raises(RuntimeError, match="lost one of its workgroups"):
+            h.step(1.0 / 60.0)
+            h.step(1.0 / 60.0) if ask == "next step" and not name.endswith("tol") else None
+            torch.cuda.synchronize()
+            stats(h) if ask == "stats" else h.step(1.0 / 60.0)
+        state = g.pos.cpu().numpy(), g.vel.cpu().numpy()
+        outs = []
+        for mode, want in ((None, "streaming"), (-1, form), (0, "streaming")):
+            if mode is not None:
+                h.set_resident_solve(mode)
+            g.pos.copy_(torch.as_tensor(state[0]))
+            g.vel.copy_(torch.as_tensor(state[1]))
+            if name != "batch":
+                h.set_warm_start(np.zeros((g.scene.n, 3)))
+            h.step(1.0 / 60.0)
+            stats(h)
+            assert h.solve_form() == want
+            outs.append(g.pos.cpu().numpy())
+        if name != "batch":
+            np.testing.assert_array_equal(outs[1], outs[0])
+            np.testing.assert_array_equal(outs[2], outs[0])
