@@ -505,6 +505,7 @@ void Problem::make_resident(const std::vector<int>& cols) {
     res_ = ResidentView{};
     res_min_iters_ = 0;
     res_lost_ = false;
+    hold_ = ResidentHold();
     sweep_ = SweepView{};
     int dev = 0, cus = 0, lds = 0;
     check_hip(hipGetDevice(&dev), "hipGetDevice");
@@ -608,9 +609,10 @@ void Problem::make_sweep(const std::vector<int>& cols, int max_wgs, int lds) {
     sweep_.groups = P.groups;
 }
 
-void Problem::launch_sweep(hipStream_t s) {
+void Problem::launch_sweep(hipStream_t s, bool waits) {
     SweepView R = sweep_;
-    if (res_mode_ == 2) R.meet_polls = 0;
+    if (res_mode_ == 2 || res_mode_ == 3) R.meet_polls = 0;
+    if (waits && res_mode_ != 2) R.solo = nullptr;
     const LaunchGeom g = geom();
     with_resident_gate(gated(), s, [&] { launch_pcg_sweep(R, g, matrix(), vectors(), state_.data(), params_.data(), s); });
     bool checks = false;
@@ -621,9 +623,11 @@ void Problem::launch_sweep(hipStream_t s) {
     launch_pcg_advance(state_.data(), params_.data(), partials_.data(), ninst_, g.ngroups, s, g.gactive);
 }
 
-void Problem::launch_resident(float dt, const DevExt& ext, hipStream_t s) {
+void Problem::launch_resident(float dt, const DevExt& ext, hipStream_t s, bool waits) {
     ResidentView R = res_;
-    if (res_mode_ == 2) R.meet_polls = 0;
+    if (res_mode_ == 2 || res_mode_ == 3) R.meet_polls = 0;
+    // the cloths of a batch that have met are solved, so the others are, too
+    if (waits && ninst_ == 1 && res_mode_ != 2) R.solo = nullptr;
     const int given_r = start_r_ready_ ? 1 : 0;
     start_r_ready_ = false;
     with_resident_gate(gated(), s, [&] {
@@ -632,16 +636,31 @@ void Problem::launch_resident(float dt, const DevExt& ext, hipStream_t s) {
     });
 }
 
-Problem::SolveForm Problem::next_form(int iters) const {
-    if (res_mode_ == 0 || res_lost_ || (res_mode_ == -1 && iters < res_min_iters_)) return kFormStreaming;
+bool Problem::not_met() {
+    volatile int* left = &notice_->left;
+    if (*left == 0) return false;
+    *left = 0;
+    hold_.missed();
+    return true;
+}
+
+Problem::SolveForm Problem::next_form(int iters) {
+    volatile int* alone = &notice_->alone;
+    if (*alone != 0) {
+        *alone = 0;
+        if (res_mode_ != 2) hold_.missed();
+    }
+    if (res_mode_ == 0 || res_lost_ || (res_.variant == kResidentNone && sweep_.groups == 0)) return kFormStreaming;
+    if (res_mode_ == -1 && iters < res_min_iters_) return kFormStreaming;
+    if (!hold_.may_run()) return kFormStreaming;
     return res_.variant != kResidentNone ? kFormResident : sweep_.groups != 0 ? kFormSweep : kFormStreaming;
 }
 
 void Problem::set_resident_solve(int mode) {
-    if (mode != -1 && mode != 0 && mode != 2 && mode != 4)
-        throw std::invalid_argument("resident solve: -1, 0, 2 or 4");
+    if (mode < -1 || mode > 4 || mode == 1) throw std::invalid_argument("resident solve: -1, 0, 2, 3 or 4");
     if (mode != 0 && (res_lost_ || mode == 4)) clear_exchange(mode == 4 ? 1u : 0u);
     res_mode_ = mode;
+    hold_ = ResidentHold();
     destroy_graph();
 }
 
@@ -1234,7 +1253,7 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
         fixed = fixed && q.tol2 == 0.0;
         fixed_iters = std::max(fixed_iters, q.max_iter);
     }
-    const SolveForm form = next_form(fixed || last_iters_ <= 0 ? fixed_iters : std::min(last_iters_, fixed_iters));
+    SolveForm form = next_form(fixed || last_iters_ <= 0 ? fixed_iters : std::min(last_iters_, fixed_iters));
     if (form != kFormStreaming) {
         // the solve is launched directly, not as a graph, so a capture is refused here
         hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
@@ -1252,13 +1271,13 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
         const int chunks = std::max(1, (fixed_iters + 2 + kChunkIters - 1) / kChunkIters);
         if (form == kFormResident) {
             launch_assemble(dt, ext, s);
-            launch_resident(dt, ext, s);
+            launch_resident(dt, ext, s, false);
         } else if (form == kFormStreaming && chunks <= kStepGraphMaxChunks) {
             launch_fixed_step_graph(dt, ext, chunks, s);
         } else {
             launch_assemble(dt, ext, s);
             launch_pcg_start(s);
-            if (form == kFormSweep) launch_sweep(s);
+            if (form == kFormSweep) launch_sweep(s, false);
             else launch_pcg_chunks(s, chunks);
             launch_pcg_residual(geom(), matrix(), vectors(), state_.data(), 1, s);
             launch_pcg_reduce(state_.data(), params_.data(), partials_.data(), ninst_, geom().ngroups, kPhaseFinal,
@@ -1280,14 +1299,19 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
     launch_assemble(dt, ext, s);
     if (ws_on && hist_n_ >= 2) warm_start_stage(dt, ext, s);
     if (form == kFormResident) {
-        launch_resident(dt, ext, s);
+        const bool given_r = start_r_ready_;
+        launch_resident(dt, ext, s, true);
         check_hip(hipStreamSynchronize(s), "hipStreamSynchronize(solve)");
         raise_if_lost();
-        last_iters_ = 0;
-        for (int k = 0; k < ninst_; ++k) last_iters_ = std::max(last_iters_, host_states_[k].iters);
-        train_after_solve(ws_on, s);
-        end_step(s);
-        return;
+        if (!not_met()) {
+            last_iters_ = 0;
+            for (int k = 0; k < ninst_; ++k) last_iters_ = std::max(last_iters_, host_states_[k].iters);
+            train_after_solve(ws_on, s);
+            end_step(s);
+            return;
+        }
+        start_r_ready_ = given_r;
+        form = form_ = kFormStreaming;
     }
     launch_pcg_start(s);
     // Launch as many rounds as the previous step used (its iterations plus a
@@ -1296,10 +1320,14 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
     int chunks = std::max(1, (last_iters_ + 2 + kChunkIters - 1) / kChunkIters);
     int guard = 0;
     for (;;) {
-        if (form == kFormSweep) launch_sweep(s);
+        if (form == kFormSweep) launch_sweep(s, true);
         else launch_pcg_chunks(s, chunks);
         read_states(s);
         raise_if_lost();
+        if (form == kFormSweep && not_met()) {
+            form = form_ = kFormStreaming;
+            continue;
+        }
         if (all_done()) break;
         chunks = 1;
         if (++guard > (1 << 22)) throw std::runtime_error("PCG did not terminate");

@@ -304,6 +304,9 @@ public:
     // -1 where it fits, 0 never, 2 where it fits but with a start-up wait of
     // no length, so that an instance's first workgroup solves it alone (for
     // tests).  Results are the same bits.
+    // 3: where it fits, with a start-up wait of no length, treated as one that
+    // ran out: a step that waits for the solve of a single cloth goes over to
+    // the streaming kernels, and they keep the next steps (for tests).
     // 4: where it fits, with the exchange between workgroups marked as one
     // that has lost a workgroup leaves it (for tests).  After a step has failed
     // for that reason the streaming kernels take over until this is called.
@@ -345,12 +348,15 @@ private:
     void make_done_event();
     GatedLaunch gated() const { return GatedLaunch{this, done_event_, gate_device_, gate_weight_, gate_room_}; }
     // The iterations of a started solve until its next true-residual check,
-    // and that check; no host wait.
-    void launch_sweep(hipStream_t s);
+    // and that check; no host wait.  waits: the caller waits and goes on with
+    // the streaming kernels where not_met() says so.
+    void launch_sweep(hipStream_t s, bool waits);
     // Assembly and the resident solve, which ends with finalize; no host wait.
-    void launch_resident(float dt, const DevExt& ext, hipStream_t s);
+    void launch_resident(float dt, const DevExt& ext, hipStream_t s, bool waits);
+    // Whether the launch that the host has waited for left the solve to it.
+    bool not_met();
     // The form of the next step's solve, of about `iters` iterations.
-    SolveForm next_form(int iters) const;
+    SolveForm next_form(int iters);
     // Throws when a solve since the last call lost a workgroup, or was not
     // started after one that did.
     void raise_if_lost() const;
@@ -411,6 +417,7 @@ private:
     int res_mode_ = -1;
     mutable bool res_lost_ = false;  // a solve lost a workgroup: the exchange words are in no known state
     ResidentNotice* notice_ = nullptr;  // behind host_states_
+    ResidentHold hold_;
     SolveForm form_ = kFormStreaming;  // of the latest step
     int res_min_iters_ = 0;  // as ResidentPlan
     ResidentView res_{};

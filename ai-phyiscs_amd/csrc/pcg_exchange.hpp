@@ -100,19 +100,23 @@ __device__ __forceinline__ double slot_wait(const Cluster& C, const u64* w, unsi
 }
 
 // A wait of the exchange ran out, in this launch or an earlier one.
+__device__ __forceinline__ void notify(int* word) {
+    __hip_atomic_store(word, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 __device__ __forceinline__ void lost_exchange(ResidentSync* S) {
     S->lost = 1;
-    __hip_atomic_store(&S->notice->lost, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    notify(&S->notice->lost);
 }
 
 // The instance's workgroups agree that they run: all of them have started, so
 // every wait that follows ends.  If they have not met within R.meet_polls (the
 // device's compute units are held by waiting workgroups of another process),
-// one of them solves the instance alone and the others leave.  After a launch
+// one of them solves the instance alone and the others leave, or all leave
+// where the caller goes on (`alone` false).  After a launch
 // that lost a workgroup all leave (a loss in this launch comes after all have
 // met, so they agree on that, too).
 enum Meeting : int { kMeetRun = 0, kMeetLeave = 1, kMeetAlone = 2 };
-__device__ int meet(ResidentSync* S, int cluster, int polls) {
+__device__ int meet(ResidentSync* S, int cluster, int polls, bool alone) {
     if (S->lost != 0) {
         lost_exchange(S);
         return kMeetLeave;
@@ -133,8 +137,10 @@ __device__ int meet(ResidentSync* S, int cluster, int polls) {
     }
     u64 old = agent_load(&S->decision);
     if (old < run && __hip_atomic_compare_exchange_strong(&S->decision, &old, run + 1, __ATOMIC_RELAXED,
-                                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        return kMeetAlone;
+                                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+        notify(alone ? &S->notice->alone : &S->notice->left);
+        return alone ? kMeetAlone : kMeetLeave;
+    }
     return old == run ? kMeetRun : kMeetLeave;
 }
 

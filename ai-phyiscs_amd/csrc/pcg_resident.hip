@@ -331,7 +331,7 @@ __global__ __launch_bounds__(64 * NW) void pcg_resident_kernel(ResidentView R, L
     unsigned tag = 0;
     if (W.cluster > 1) {
         tag = R.sync[W.inst].epoch;
-        if (tid == 0) shared_int[1] = meet(R.sync + W.inst, W.cluster, R.meet_polls);
+        if (tid == 0) shared_int[1] = meet(R.sync + W.inst, W.cluster, R.meet_polls, R.solo != nullptr);
     } else if (tid == 0) {
         shared_int[1] = kMeetRun;
     }

@@ -153,7 +153,36 @@ ResidentPlan plan_resident(const std::vector<ResidentInstance>& insts, const std
 // What the host has to know of solves that it may not ask for their outcome,
 // in pinned memory; stays until the host takes it back.
 struct ResidentNotice {
-    int lost;  // 1: a solve lost a workgroup, or was not started after one that did
+    int lost;   // 1: a solve lost a workgroup, or was not started after one that did
+    int alone;  // 1: an instance's workgroups did not meet in time, and one of them solved it
+    int left;   // 1: the same of a launch that leaves the solve to the caller
+};
+
+// Steps on the streaming kernels after a solve whose workgroups did not meet
+// in time: something else holds compute units (another process, a mask), and
+// each try costs the start-up bound and, where the host does not wait for the
+// solve, one by a single workgroup (up to a second or more).  1024 steps, then
+// twice as many each time, until as many have met.
+class ResidentHold {
+public:
+    static constexpr int kFirst = 1024, kLongest = 1 << 16;
+    // Called once a step: whether it may be solved in one launch.
+    bool may_run() {
+        if (left_ > 0) {
+            --left_;
+            return false;
+        }
+        if (++met_ > next_) next_ = kFirst;
+        return true;
+    }
+    void missed() {
+        left_ = next_;
+        next_ = std::min(2 * next_, kLongest);
+        met_ = 0;
+    }
+
+private:
+    int left_ = 0, next_ = kFirst, met_ = 0;
 };
 
 // Start-up agreement of an instance's workgroups, kept in device memory across
@@ -177,7 +206,8 @@ struct ResidentView {
     unsigned long long* zx;     // 2 words a row (all first words, then all second ones): z of the exported rows
     int rows;                   // padded rows of the problem
     unsigned long long* slots;  // partial sums: kinds x pieces x copies x 2 halves x groups words
-    double* solo;               // 3 per slice: partial sums of an instance solved by one workgroup
+    double* solo;               // 3 per slice: partial sums of an instance solved by one workgroup;
+                                // null: a launch whose workgroups do not meet leaves all as it was
     ResidentSync* sync;         // per instance
     unsigned long long* ticket; // workgroups started, over all launches; null: places by number
     int meet_polls;             // bound of the start-up wait, in polls of about a microsecond

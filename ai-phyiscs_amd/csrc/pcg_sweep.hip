@@ -208,7 +208,7 @@ __global__ __launch_bounds__(kThreads) void pcg_sweep_kernel(SweepView R, Launch
     unsigned tag = R.sync->epoch;
     if (tid == 0) {
         sh.failed = 0;
-        sh.met = meet(R.sync, R.nwg, R.meet_polls);
+        sh.met = meet(R.sync, R.nwg, R.meet_polls, R.solo != nullptr);
     }
     __syncthreads();
     const int met = uniform_int(sh.met);

@@ -56,7 +56,7 @@ struct SweepView {
     const uint8_t* exported;
     unsigned long long* zx;     // as ResidentView
     unsigned long long* slots;  // kinds x copies x 2 halves x groups words
-    double* solo;               // 3 per slice
+    double* solo;               // 3 per slice, or null
     ResidentSync* sync;
     int meet_polls;
     int pause;  // before the look for p . Ap; the update's sums wait behind the iterate and need none

@@ -200,6 +200,11 @@ int chysx_cloth_set_pin_projection(chysx_cloth* sim, int on);
  * regularly triangulated cloth up to 1024x1024, its vectors; 0: always in
  * the kernels that stream the matrix; 2: as -1, with a start-up wait of no
  * length, after which one workgroup solves alone (tests).  Same bits.
+ * Where the workgroups of a solve do not all start within half a second
+ * (another process holds compute units), a step that waits for the solve of
+ * one cloth streams the matrix, otherwise one workgroup solves alone; the next
+ * 1024 steps, and more if it happens again, stream.  3: as -1, with a start-up
+ * wait of no length (tests).
  * A solve whose workgroups lose each other ends after some seconds, and the
  * step, the statistics or the next step report it as an error; later steps
  * stream the matrix until this is called again.  4: as -1, marked as such a

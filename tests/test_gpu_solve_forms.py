@@ -270,3 +270,48 @@ def test_lost_workgroup_is_reported_and_not_trusted(cuda, name):
         if name != "batch":
             np.testing.assert_array_equal(outs[1], outs[0])
             np.testing.assert_array_equal(outs[2], outs[0])
+
+
+def learned():
+    from chysx.warmstart import load_params
+    g = make_sim(mesh(130), tol=1e-6)
+    g.sim.ws_set_params(load_params()[0])
+    g.sim.set_warm_start_mode("learned")
+    return g
+
+
+# name: what is solved, the form of the step whose workgroups do not meet (one
+# workgroup alone where the host does not wait, or in a batch), of the others
+NOT_MET = {
+    "waits": (lambda: make_sim(mesh(130), tol=1e-6), "streaming", "one_launch"),
+    "enqueued": (lambda: make_sim(mesh(130), tol=0.0, max_iter=9), "one_launch", "one_launch"),
+    "learned": (learned, "streaming", "one_launch"),
+    "batch": (lambda: make_batch([mesh(w) for w in (130, 100, 20)], tol=1e-6), "one_launch", "one_launch"),
+    "sweep_waits": (lambda: make_sim(mesh(520), tol=1e-4), "streaming", "sweep"),
+    "sweep_enqueued": (lambda: make_sim(mesh(520), tol=0.0, max_iter=3), "sweep", "sweep"),
+}
+
+
+@pytest.mark.parametrize("name", NOT_MET)
+def test_workgroups_that_do_not_meet(cuda, name):
+    """A start-up wait of no length (mode 3), from the fourth step on: that step
+    gives the same bits, the next ones stream, and the one-launch form comes
+    back when it is asked for."""
+    import torch
+    make, missed, form = NOT_MET[name]
+    outs = []
+    for mode in (0, 3):
+        g = make()
+        h = handle(g)
+        rows, forms = [], []
+        for k in range(8):
+            if k in (0, 3, 6):
+                h.set_resident_solve(0 if mode == 0 else {0: -1, 3: 3, 6: -1}[k])
+            h.step(1.0 / 60.0)
+            torch.cuda.synchronize()
+            forms.append(h.solve_form())
+            rows += [g.pos.cpu().numpy(), g.vel.cpu().numpy()]
+        outs.append(rows)
+        assert forms == (["streaming"] * 8 if mode == 0 else [form] * 3 + [missed] + ["streaming"] * 2 + [form] * 2)
+    for a, b in zip(*outs):
+        np.testing.assert_array_equal(a, b)

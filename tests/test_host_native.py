@@ -49,3 +49,8 @@ def test_batches_that_the_streaming_kernels_solve_faster(compiled):
 def test_solves_in_flight_together_leave_room(compiled):
     """Launches that may be under way together never hold a whole XCD with waiting workgroups."""
     assert compiled("gate").startswith("ok ")
+
+
+def test_steps_held_after_workgroups_did_not_meet(compiled):
+    """None at first, then 1024 and twice as many at each miss, up to 65536; 1024 again after as many have met."""
+    assert [int(v) for v in compiled("hold").split()] == [0, 1024, 2048, 4096, 8192, 16384, 32768, 65536, 65536, 65536, 1024]
