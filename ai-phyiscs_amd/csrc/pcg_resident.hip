@@ -138,9 +138,11 @@ __device__ __forceinline__ bool cluster_sum(const Cluster& C, SumShared<NW>& sh,
             }
         }
     } else {
-        // few workgroups: the sums come soon after z (20 half groups: 2.83 ms,
-        // and 2.95 ms with z first; 176: 637 us, and 610)
-        const bool z_first = C.pause >= 18;
+        // few workgroups: the sums come soon after z.  100 iterations of a
+        // drape, sums first and z first: 20 workgroups 727 and 765 us, 64: 873
+        // and 882, 104: 906 and 929, 130: 979 and 966, 176: 1055 and 1024, 256:
+        // 1160 and 1066
+        const bool z_first = C.size >= 120;
         if (z_first) meanwhile();
         // A group's first half is one value, its second half's waves are 8:
         // a few values a thread, all loaded before any is looked at.
