@@ -6,16 +6,17 @@
 // Jacobi inverse and the diagonal blocks stay in registers, the directions of
 // its rows and of its neighbours' boundary rows in LDS, so an iteration reads
 // only the off-diagonal blocks and their packed indices (92 bytes a row and 18
-// more for mirrors that have left the L2) and, every other time, the iterate:
-// about 135 bytes a row on average against 270 of the streaming kernels, which
-// also pay two more launches.  z of the boundary rows and the sums travel as in
-// the resident solve.
+// more for mirrors that have left the L2), every other time the iterate, and z
+// of the boundary rows (16 bytes for up to half of the rows, both ways): 157
+// bytes a row counted at 1024 x 1024 against 270 of the streaming kernels,
+// which also pay two more launches.  The sums and z travel as in the resident
+// solve.
 //
 // At 1024 x 1024 an iteration takes 31 us against 53 us (about 75 K cycles: 31
 // to 36 K in the products, 15 to 22 K for p . Ap with 5 to 12 K of it waiting
 // for the slowest workgroup, 17 K for the update's sums with the iterate under
-// them), and three steps solved to 1e-6 take 10.9 ms where they took 18.7 ms.  The products
-// read 4.5 TB/s from the Infinity Cache; with 8 waves a compute unit more loads
+// them), and three steps solved to 1e-6 take 10.9 ms where they took 18.7 ms.  It
+// moves 164 MB beyond the L2, 5.4 TB/s; with 8 waves a compute unit more loads
 // in flight would need registers that the vectors hold.  Fewer, larger pieces
 // (2 groups at 512 x 512 on half the units) lose to the resident solve, and
 // rows wider than 6 entries, which would have to take a generic loop, make
