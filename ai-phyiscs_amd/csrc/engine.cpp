@@ -1254,21 +1254,28 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
         fixed_iters = std::max(fixed_iters, q.max_iter);
     }
     SolveForm form = next_form(fixed || last_iters_ <= 0 ? fixed_iters : std::min(last_iters_, fixed_iters));
+    // max_iter iterations plus a flush round and the advance that stops the
+    // solve (rounds after the stop exit at once)
+    const int fixed_chunks = std::max(1, (fixed_iters + 2 + kChunkIters - 1) / kChunkIters);
     if (form != kFormStreaming) {
-        // the solve is launched directly, not as a graph, so a capture is refused here
+        // A launch of the solve would be recorded into a capture of the stream,
+        // where no step can wait for it.  The streaming form's graph is not: it
+        // runs at once, outside the captured graph.
         hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
         check_hip(hipStreamIsCapturing(s, &capturing), "hipStreamIsCapturing");
-        if (capturing != hipStreamCaptureStatusNone)
-            throw std::runtime_error("step: the stream is being captured; a step cannot be part of a graph");
+        if (capturing != hipStreamCaptureStatusNone) {
+            if (!fixed || blocking_ || fixed_chunks > kStepGraphMaxChunks)
+                throw std::runtime_error("step: the stream is being captured; a step cannot be part of a graph");
+            form = kFormStreaming;
+        }
     }
     form_ = form;
     if (fixed && !blocking_) {
-        // max_iter iterations plus a flush round and the advance that stops
-        // the solve (rounds after the stop exit at once): the whole step,
-        // assembly to finalize and the statistics' copy, is one graph; very
-        // long fixed solves replay the chunk graphs instead, so a graph never
-        // holds more than kStepGraphMaxChunks chunks
-        const int chunks = std::max(1, (fixed_iters + 2 + kChunkIters - 1) / kChunkIters);
+        // on the streaming kernels the whole step, assembly to finalize and the
+        // statistics' copy, is one graph; very long fixed solves replay the
+        // chunk graphs instead, so a graph never holds more than
+        // kStepGraphMaxChunks chunks
+        const int chunks = fixed_chunks;
         if (form == kFormResident) {
             launch_assemble(dt, ext, s);
             launch_resident(dt, ext, s, false);

@@ -315,3 +315,49 @@ def test_workgroups_that_do_not_meet(cuda, name):
         assert forms == (["streaming"] * 8 if mode == 0 else [form] * 3 + [missed] + ["streaming"] * 2 + [form] * 2)
     for a, b in zip(*outs):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("w", [20, 60, 530])
+def test_step_on_a_stream_that_is_being_captured(cuda, w):
+    """A fixed-count step with nothing enqueued before it runs at once, outside
+    the captured graph; one that waits for its solve is refused and changes
+    nothing."""
+    import torch
+    kw = dict(tol=0.0, max_iter=20)
+    ref = make_sim(mesh(w), **kw)
+    want = []
+    for _ in range(4):
+        ref.sim.step(1.0 / 60.0)
+        want.append(ref.positions())
+    g = make_sim(mesh(w), **kw)
+    s = torch.cuda.Stream()
+    g.sim.step(1.0 / 60.0, s.cuda_stream)
+    assert g.sim.last_solve_stats()["iters"] == 20
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        x = torch.zeros(8, device="cuda")
+        g.sim.step(1.0 / 60.0, s.cuda_stream)
+        x += 1
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(g.positions(), want[1])
+    assert g.sim.last_solve_stats()["iters"] == 20
+    for _ in range(2):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert (x == 1).all()
+    np.testing.assert_array_equal(g.positions(), want[1])
+    g.sim.step(1.0 / 60.0, s.cuda_stream)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(g.positions(), want[2])
+    assert g.sim.last_solve_stats()["iters"] == 20
+    g.sim.set_blocking_step(True)
+    other = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(other, stream=s):
+        x = torch.zeros(8, device="cuda")
+        with pytest.raises(RuntimeError, match="being captured"):
+            g.sim.step(1.0 / 60.0, s.cuda_stream)
+    other.replay()
+    g.sim.step(1.0 / 60.0, s.cuda_stream)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(g.positions(), want[3])
