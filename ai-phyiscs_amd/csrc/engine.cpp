@@ -1267,6 +1267,9 @@ void Problem::step(float dt, const DevExt& ext, hipStream_t s) {
             if (!fixed || blocking_ || fixed_chunks > kStepGraphMaxChunks)
                 throw std::runtime_error("step: the stream is being captured; a step cannot be part of a graph");
             form = kFormStreaming;
+            // the solves before have run (the wait above is refused otherwise),
+            // and the event, recorded into the capture, says nothing of them
+            leave_resident_gate(gate_device_, this);
         }
     }
     form_ = form;

@@ -361,3 +361,29 @@ def test_step_on_a_stream_that_is_being_captured(cuda, w):
     g.sim.step(1.0 / 60.0, s.cuda_stream)
     torch.cuda.synchronize()
     np.testing.assert_array_equal(g.positions(), want[3])
+
+
+def test_other_solves_beside_a_step_on_a_captured_stream(cuda):
+    """A step that runs at once on a stream under capture leaves the other
+    cloths' solves on other streams as they are."""
+    import torch
+    kw = dict(tol=0.0, max_iter=20)
+    ref = make_sim(mesh(130), **kw)
+    for _ in range(3):
+        ref.sim.step(1.0 / 60.0)
+    a, b = make_sim(mesh(130), **kw), make_sim(mesh(130), **kw)
+    s, t = torch.cuda.Stream(), torch.cuda.Stream()
+    for g, q in ((a, s), (b, t)):
+        g.sim.step(1.0 / 60.0, q.cuda_stream)
+        g.sim.last_solve_stats()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        x = torch.zeros(8, device="cuda")
+        a.sim.step(1.0 / 60.0, s.cuda_stream)
+    b.sim.step(1.0 / 60.0, t.cuda_stream)
+    b.sim.step(1.0 / 60.0, t.cuda_stream)
+    a.sim.step(1.0 / 60.0, s.cuda_stream)
+    torch.cuda.synchronize()
+    for g in (a, b):
+        np.testing.assert_array_equal(g.positions(), ref.positions())
